@@ -33,31 +33,20 @@ MF_HD C2<T> rotq(C2<T> a)
     return {a.y, -a.x};
 }
 
-// cos(k pi / 8) for k = 0..4
-constexpr double kC0 = 1.0;
-constexpr double kC1 = 0.92387953251128675613;  // cos(pi/8)
-constexpr double kC2 = 0.70710678118654752440;  // cos(pi/4)
-constexpr double kC3 = 0.38268343236508977173;  // cos(3pi/8)
+constexpr double kCos8 = 0.92387953251128675613;   // cos(pi/8)
+constexpr double kTan8 = 0.41421356237309504880;   // tan(pi/8)
+constexpr double kHalfRt = 0.70710678118654752440; // cos(pi/4)
 
-// W16^e = exp(-+ 2 pi i e / 16) for e in [0, 16) (sign by INV)
+// a (1 -+ i t) (sign by INV): a rotation by -+ atan(t) up to the factor
+// cos(atan(t)), which the caller folds into its next additions.
 template <bool INV, typename T>
-MF_HD C2<T> w16(int e)
+MF_HD C2<T> rotT(C2<T> a, T t)
 {
-    // cos/sin of 2 pi e/16 from the first-quadrant constants
-    const double cs[5] = {kC0, kC1, kC2, kC3, 0.0};
-    const int q = e & 3;          // position inside the quadrant (units of pi/8)
-    const int quad = (e >> 2) & 3;
-    double c = cs[q], s = cs[4 - q];
-    double cr, sr;
-    switch (quad) {
-    case 0: cr = c; sr = s; break;
-    case 1: cr = -s; sr = c; break;
-    case 2: cr = -c; sr = -s; break;
-    default: cr = s; sr = -c; break;
-    }
-    // forward twiddle exp(-i theta) = (cos, -sin)
-    return {static_cast<T>(cr), static_cast<T>(INV ? sr : -sr)};
+    if constexpr (INV) { return {a.x - t * a.y, a.y + t * a.x}; }
+    return {a.x + t * a.y, a.y - t * a.x};
 }
+template <typename T>
+MF_HD C2<T> addScaled(C2<T> a, T c, C2<T> b) { return {a.x + c * b.x, a.y + c * b.y}; }
 
 template <bool INV, typename T>
 MF_HD void dft4(C2<T> &a0, C2<T> &a1, C2<T> &a2, C2<T> &a3)
@@ -70,6 +59,20 @@ MF_HD void dft4(C2<T> &a0, C2<T> &a1, C2<T> &a2, C2<T> &a3)
     a3 = sub(t1, t3);
 }
 
+// Second stage of the radix-8 and radix-16 codelets: a 4-point DFT of
+// a0, c2 a2 and c a1, c a3 with real factors c, c2 left over by rotT.  The
+// factors ride on the additions as fused multiply-adds.
+template <bool INV, typename T>
+MF_HD void dft4Scaled(C2<T> &a0, C2<T> &a1, C2<T> &a2, C2<T> &a3, T c, T c2)
+{
+    const C2<T> t0 = addScaled(a0, c2, a2), t1 = addScaled(a0, -c2, a2);
+    const C2<T> t2 = add(a1, a3), t3 = rotq<INV>(sub(a1, a3));
+    a0 = addScaled(t0, c, t2);
+    a2 = addScaled(t0, -c, t2);
+    a1 = addScaled(t1, c, t3);
+    a3 = addScaled(t1, -c, t3);
+}
+
 // 8-point DFT in place (natural order in and out).
 template <bool INV, typename T>
 MF_HD void dft8(C2<T> *v)
@@ -78,29 +81,26 @@ MF_HD void dft8(C2<T> *v)
     C2<T> o0 = v[1], o1 = v[3], o2 = v[5], o3 = v[7];
     dft4<INV>(e0, e1, e2, e3);
     dft4<INV>(o0, o1, o2, o3);
-    const T h = static_cast<T>(kC2);
-    // W8^1, W8^2, W8^3
-    C2<T> p1, p2, p3;
-    if constexpr (INV) {
-        p1 = {h * (o1.x - o1.y), h * (o1.x + o1.y)};
-        p2 = {-o2.y, o2.x};
-        p3 = {-h * (o3.x + o3.y), h * (o3.x - o3.y)};
-    } else {
-        p1 = {h * (o1.x + o1.y), h * (o1.y - o1.x)};
-        p2 = {o2.y, -o2.x};
-        p3 = {h * (o3.y - o3.x), -h * (o3.x + o3.y)};
-    }
+    const T h = static_cast<T>(kHalfRt);
+    // W8^1 o1 and W8^3 o3 without their factor h, W8^2 o2
+    const C2<T> p1 = rotT<INV>(o1, T(1));
+    const C2<T> p2 = rotq<INV>(o2);
+    const C2<T> p3 = rotq<INV>(rotT<INV>(o3, T(1)));
     v[0] = add(e0, o0);
     v[4] = sub(e0, o0);
-    v[1] = add(e1, p1);
-    v[5] = sub(e1, p1);
+    v[1] = addScaled(e1, h, p1);
+    v[5] = addScaled(e1, -h, p1);
     v[2] = add(e2, p2);
     v[6] = sub(e2, p2);
-    v[3] = add(e3, p3);
-    v[7] = sub(e3, p3);
+    v[3] = addScaled(e3, h, p3);
+    v[7] = addScaled(e3, -h, p3);
 }
 
 // 16-point DFT in place: 4 x 4 decomposition (n = 4 n1 + n2, k = k1 + 4 k2).
+// The inner twiddles W16^e are tangent rotations (e = 1, 3, 9 by pi/8 up to
+// quarter turns, e = 2, 6 by pi/4, e = 4 a quarter turn) whose cosines ride
+// on the second stage's additions: 144 instructions instead of 164 with
+// full complex products.
 template <bool INV, typename T>
 MF_HD void dft16(C2<T> *v)
 {
@@ -113,19 +113,29 @@ MF_HD void dft16(C2<T> *v)
         a[n2][3] = v[12 + n2];
         dft4<INV>(a[n2][0], a[n2][1], a[n2][2], a[n2][3]);
     }
-#pragma unroll
-    for (int n2 = 1; n2 < 4; ++n2) {
-#pragma unroll
-        for (int k1 = 1; k1 < 4; ++k1) { a[n2][k1] = mul(a[n2][k1], w16<INV, T>(n2 * k1)); }
-    }
+    const T t = static_cast<T>(kTan8), c = static_cast<T>(kCos8), h = static_cast<T>(kHalfRt);
+    // k1 = 1: W^1, W^2, W^3 = -i W^-1 (forward)
+    a[1][1] = rotT<INV>(a[1][1], t);
+    a[2][1] = rotT<INV>(a[2][1], T(1));
+    a[3][1] = rotq<INV>(rotT<!INV>(a[3][1], t));
+    // k1 = 2: W^2, W^4 = -i, W^6 = -i W^2
+    a[1][2] = rotT<INV>(a[1][2], T(1));
+    a[2][2] = rotq<INV>(a[2][2]);
+    a[3][2] = rotq<INV>(rotT<INV>(a[3][2], T(1)));
+    // k1 = 3: W^3, W^6, W^9 = -W^1
+    a[1][3] = rotq<INV>(rotT<!INV>(a[1][3], t));
+    a[2][3] = rotq<INV>(rotT<INV>(a[2][3], T(1)));
+    a[3][3] = rotT<INV>(C2<T>{-a[3][3].x, -a[3][3].y}, t);
+    dft4<INV>(a[0][0], a[1][0], a[2][0], a[3][0]);
+    dft4Scaled<INV>(a[0][1], a[1][1], a[2][1], a[3][1], c, h);
+    dft4Scaled<INV>(a[0][2], a[1][2], a[2][2], a[3][2], h, T(1));
+    dft4Scaled<INV>(a[0][3], a[1][3], a[2][3], a[3][3], c, h);
 #pragma unroll
     for (int k1 = 0; k1 < 4; ++k1) {
-        C2<T> b0 = a[0][k1], b1 = a[1][k1], b2 = a[2][k1], b3 = a[3][k1];
-        dft4<INV>(b0, b1, b2, b3);
-        v[k1] = b0;
-        v[k1 + 4] = b1;
-        v[k1 + 8] = b2;
-        v[k1 + 12] = b3;
+        v[k1] = a[0][k1];
+        v[k1 + 4] = a[1][k1];
+        v[k1 + 8] = a[2][k1];
+        v[k1 + 12] = a[3][k1];
     }
 }
 

@@ -2,16 +2,24 @@
 //
 // FFTs are Stockham auto-sort transforms executed in LDS: each pass reads
 // a thread's butterflies into registers, synchronises, applies twiddles and
-// a radix-4 (or a final radix-2) DFT and writes back in place.  Real
-// transforms of N = 2M samples use one M-point complex transform plus the
-// even/odd packing identities; the correlation kernel folds the unpacking,
-// the product with the template spectrum and the inverse packing into one
-// LDS pass.
+// a radix-4 (or a final radix-2) DFT and writes back in place.
 //
-// Twiddles W_{2M}^e = exp(-2 pi i e / 2M) come from a two-level table
-// (64 low entries x 2M/64 high entries, computed in FP64 on the host with
-// the C library's cos/sin and rounded to T), so one complex product gives
-// any twiddle to about one ulp.
+// The correlation of a block of N = 2M real samples is taken modulo
+// z^N + 1 (its outputs before the wrap-around are the linear correlation's,
+// as with z^N - 1).  z^N + 1 = (z^M + i)(z^M - i), and the second factor's
+// residue is the conjugate of the first's, so a real block x is carried by
+// the M complex values
+//     u_j = (x_j - i x_{j+M}) W_{4M}^j,   W_{4M} = exp(-2 pi i / 4M),
+// whose M-point transform U_k holds x at the roots exp(-2 pi i (k+1/4)/M) of
+// z^M = -i.  The spectrum of the correlation with a template is U_k H_k, H_k
+// the conjugate of the template's own transform over M, with no pairing of
+// bins, and its inverse transform times W_{4M}^-n is c_n - i c_{n+M}.  The
+// packing of even and odd samples that a transform of z^N - 1 needs (split
+// and merge of bins k and M - k around every product) has no counterpart.
+//
+// Twiddles W_{4M}^e come from a two-level table (64 low entries x 4M/64 high
+// entries, computed in FP64 on the host with the C library's cos/sin and
+// rounded to T), so one complex product gives any twiddle to about one ulp.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -55,20 +63,16 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(void *p, int bytes
 {
     return __builtin_amdgcn_make_buffer_rsrc(p, 0, bytes, 0x00020000);
 }
-__device__ __forceinline__ void buffer_store_pair(float x, float y, __amdgpu_buffer_rsrc_t r, int byteOff)
+__device__ __forceinline__ void buffer_store(float x, __amdgpu_buffer_rsrc_t r, int byteOff)
+{
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x), r, byteOff, 0, 0);
+}
+__device__ __forceinline__ void buffer_store(double x, __amdgpu_buffer_rsrc_t r, int byteOff)
 {
     typedef unsigned int u2 __attribute__((ext_vector_type(2)));
-    const u2 d = {__float_as_uint(x), __float_as_uint(y)};
-    __builtin_amdgcn_raw_buffer_store_b64(d, r, byteOff, 0, 0);
-}
-__device__ __forceinline__ void buffer_store_pair(double x, double y, __amdgpu_buffer_rsrc_t r, int byteOff)
-{
-    typedef unsigned int u4 __attribute__((ext_vector_type(4)));
     const unsigned long long a = static_cast<unsigned long long>(__double_as_longlong(x));
-    const unsigned long long b = static_cast<unsigned long long>(__double_as_longlong(y));
-    const u4 d = {static_cast<unsigned>(a), static_cast<unsigned>(a >> 32), static_cast<unsigned>(b),
-                  static_cast<unsigned>(b >> 32)};
-    __builtin_amdgcn_raw_buffer_store_b128(d, r, byteOff, 0, 0);
+    const u2 d = {static_cast<unsigned>(a), static_cast<unsigned>(a >> 32)};
+    __builtin_amdgcn_raw_buffer_store_b64(d, r, byteOff, 0, 0);
 }
 
 template <typename T>
@@ -92,8 +96,8 @@ __device__ __forceinline__ Cx<T> cmulmi(Cx<T> a) { return {a.y, -a.x}; }
 // Two-level twiddle table resident in LDS.
 template <typename T>
 struct Twiddle {
-    const Cx<T> *lo;  // W_{2M}^i,       i < 64
-    const Cx<T> *hi;  // W_{2M}^(64 j),  j < 2M/64
+    const Cx<T> *lo;  // W_{4M}^i,       i < 64
+    const Cx<T> *hi;  // W_{4M}^(64 j),  j < 4M/64
     __device__ __forceinline__ Cx<T> operator()(int e) const { return cmul(lo[e & 63], hi[e >> 6]); }
 };
 
@@ -141,8 +145,8 @@ __device__ __forceinline__ void stockham_pass(Cx<T> *buf, int Ns, Twiddle<T> tw)
         const int j = t + b * NT;
         if (NB % NT == 0 || j < NB) {
             const int k = j & (Ns - 1);
-            // W_{Ns R}^{r k} = W_{2M}^{r * 2k M / (Ns R)}
-            const int step = 2 * (M / (Ns * R)) * k;
+            // W_{Ns R}^{r k} = W_{4M}^{r * 4k M / (Ns R)}
+            const int step = 4 * (M / (Ns * R)) * k;
 #pragma unroll
             for (int r = 1; r < R; ++r) {
                 Cx<T> w = tw(r * step);
@@ -296,60 +300,118 @@ __device__ __forceinline__ void wave_load(Cx<T> *v, const Cx<T> *buf, int lane)
     }
 }
 
-// Inter-pass twiddles of one lane.  They depend on the lane only (not on
-// the data or the template row), so a block computes them once and every
-// transform reuses them (conjugated for inverse transforms).
-//   pass 2: butterfly j has k = j mod R1 = lane mod R1 (64 is a multiple
-//           of R1), the same for all of the lane's butterflies;
-//   pass 3: k = j mod R1 R2, which differs per butterfly when R1 R2 > 64.
-// W3REG: pass-3 twiddle rows resident in registers (computed once per
-// block); otherwise looked up from the two-level table per transform, which
-// saves registers where they limit occupancy.
+// cos and sin of 2 pi num / den at compile time (Taylor series around 0
+// after reduction to an eighth of a turn).
+constexpr double turnSeries(double x, bool sine)
+{
+    double term = sine ? x : 1.0, sum = term;
+    for (int k = sine ? 2 : 1; k < 24; k += 2) {
+        term = -term * x * x / (k * (k + 1));
+        sum += term;
+    }
+    return sum;
+}
+constexpr double turnCos(int num, int den)
+{
+    num %= den;
+    if (num < 0) { num += den; }
+    if (2 * num > den) { num = den - num; }           // cos(-a) = cos(a)
+    const bool neg = 4 * num > den;                   // cos(pi - a) = -cos(a)
+    const int m = neg ? den - 2 * num : 2 * num;      // half turns: angle = pi m / den
+    const double pi = 3.14159265358979323846;
+    const double c = 4 * m <= den ? turnSeries(pi * m / den, false)
+                                  : turnSeries(pi * (den - 2 * m) / (2 * den), true);
+    return neg ? -c : c;
+}
+constexpr double turnSin(int num, int den) { return turnCos(4 * num - den, 4 * den); }
+
+// Inter-pass twiddles of one lane's inverse transforms.  They depend on the
+// lane only (not on the data or the template row), so a block computes them
+// once and every transform reuses them.
+//   pass 2: butterfly j has k = j mod R1 = lane mod R1 (64 is a multiple of
+//           R1), the same for all of the lane's butterflies;
+//   pass 3: element r of butterfly j = lane + 64 b gets W_M^-(j (r + 1/4)):
+//           the transform's own twiddle W_M^-(j r) and the lane part of the
+//           output weight W_{4M}^-n, n = j + m M/R3.  What is left of that
+//           weight, W_{4 R3}^-m, is the same for every lane (unweight3).
+// W3REG: a pass-3 row per butterfly in registers; otherwise one row for
+// butterfly 0 and a constant complex product per element for the others
+// (no LDS reads, and 2 (B3 - 1) R3 fewer registers).
 template <typename T, int M, bool W3REG = true>
 struct WaveTwiddles {
     using P = WavePlan<M>;
     static constexpr int NS2 = P::R1;
-    static constexpr int NS3 = P::R1 * P::R2;
     static constexpr int B3 = M / (P::R3 * 64);
     static constexpr int W3 = W3REG ? B3 : 1;
-    Cx<T> w2[P::R2 - 1];  // pass 2, resident in registers
-    Cx<T> w3[W3][P::R3 - 1];
-    Twiddle<T> tab;       // pass 3, looked up per transform
-    __device__ __forceinline__ void init(int lane, const Twiddle<T> &tw)
+    Cx<T> w2[P::R2 - 1];
+    Cx<T> w3[W3][P::R3];
+    __device__ __forceinline__ void initPass2(int lane, const Twiddle<T> &tw)
     {
-        tab = tw;
         const int k2 = lane & (NS2 - 1);
-        const int s2 = (2 * M / (NS2 * P::R2)) * k2;
+        const int s2 = (4 * M / (NS2 * P::R2)) * k2;
 #pragma unroll
-        for (int r = 1; r < P::R2; ++r) { w2[r - 1] = tw(r * s2); }
-        if constexpr (W3REG) {
-#pragma unroll
-            for (int b = 0; b < B3; ++b) { lookup3(lane, b, w3[b]); }
-        }
+        for (int r = 1; r < P::R2; ++r) { w2[r - 1] = cconj(tw(r * s2)); }
     }
-    __device__ __forceinline__ void lookup3(int lane, int b, Cx<T> *w) const
+    __device__ __forceinline__ void initPass3(int lane, const Twiddle<T> &tw)
     {
-        const int k3 = (lane + 64 * b) & (NS3 - 1);
-        const int s3 = (2 * M / (NS3 * P::R3)) * k3;
 #pragma unroll
-        for (int r = 1; r < P::R3; ++r) { w[r - 1] = tab(r * s3); }
-    }
-    // pass-3 twiddle row of butterfly b of this lane
-    __device__ __forceinline__ void pass3(int lane, int b, Cx<T> *w) const
-    {
-        if constexpr (W3REG) {
+        for (int b = 0; b < W3; ++b) {
 #pragma unroll
-            for (int r = 1; r < P::R3; ++r) { w[r - 1] = w3[b][r - 1]; }
-        } else {
-            lookup3(lane, b, w);
+            for (int r = 0; r < P::R3; ++r) { w3[b][r] = cconj(tw((lane + 64 * b) * (4 * r + 1))); }
         }
     }
 };
 
-// Butterflies of one pass with per-butterfly twiddle rows w[b][r-1]
-// (wStride 0 when all butterflies share one row).
+// exp(2 pi i NUM / DEN) as a constant of type T.
+template <typename T, int NUM, int DEN>
+__device__ __forceinline__ Cx<T> turn()
+{
+    constexpr double c = turnCos(NUM, DEN), s = turnSin(NUM, DEN);
+    return {static_cast<T>(c), static_cast<T>(s)};
+}
+
+// Pass 3 of an inverse transform: twiddles with the output weight, DFTs,
+// and the rest of the output weight.  On return v[b R3 + m] is point
+// n = lane + 64 b + m M/R3 of c_n - i c_{n+M}.
+template <int B, int R, typename T, int M, typename W>
+__device__ __forceinline__ void unweighted_twiddle(Cx<T> *v, const W &tw)
+{
+    using P = WavePlan<M>;
+    if constexpr (W::W3 > 1 || B == 0) {
+        v[B * P::R3 + R] = cmul(v[B * P::R3 + R], tw.w3[B][R]);
+    } else {
+        v[B * P::R3 + R] = cmul(v[B * P::R3 + R], cmul(tw.w3[0][R], turn<T, 16 * B * (4 * R + 1), M>()));
+    }
+    if constexpr (R + 1 < P::R3) {
+        unweighted_twiddle<B, R + 1, T, M>(v, tw);
+    } else if constexpr (B + 1 < W::B3) {
+        unweighted_twiddle<B + 1, 0, T, M>(v, tw);
+    }
+}
+template <int R, typename T, int M>
+__device__ __forceinline__ void unweight3(Cx<T> *v)
+{
+    using P = WavePlan<M>;
+    constexpr int B3 = M / (P::R3 * 64);
+#pragma unroll
+    for (int b = 0; b < B3; ++b) { v[b * P::R3 + R] = cmul(v[b * P::R3 + R], turn<T, R, 4 * P::R3>()); }
+    if constexpr (R + 1 < P::R3) { unweight3<R + 1, T, M>(v); }
+}
+template <typename T, int M, typename W>
+__device__ __forceinline__ void wave_pass3_inverse(Cx<T> *v, const W &tw)
+{
+    using P = WavePlan<M>;
+    unweighted_twiddle<0, 0, T, M>(v, tw);
+#pragma unroll
+    for (int b = 0; b < W::B3; ++b) { mfcl::dftR<P::R3, true>(&v[b * P::R3]); }
+    unweight3<1, T, M>(v);
+}
+
+// Butterflies of one pass; with TWIDDLE, element r of each is first
+// multiplied by w[r-1] (a row of inverse twiddles, conjugated for forward
+// transforms).
 template <typename T, int M, int R, bool INV, bool TWIDDLE>
-__device__ __forceinline__ void wave_butterflies(Cx<T> *v, const Cx<T> *w, int wStride)
+__device__ __forceinline__ void wave_butterflies(Cx<T> *v, const Cx<T> *w)
 {
     constexpr int B = M / (R * 64);
 #pragma unroll
@@ -357,8 +419,8 @@ __device__ __forceinline__ void wave_butterflies(Cx<T> *v, const Cx<T> *w, int w
         if constexpr (TWIDDLE) {
 #pragma unroll
             for (int r = 1; r < R; ++r) {
-                Cx<T> t = w[b * wStride + r - 1];
-                if (INV) { t.y = -t.y; }
+                Cx<T> t = w[r - 1];
+                if (!INV) { t.y = -t.y; }
                 v[b * R + r] = cmul(v[b * R + r], t);
             }
         }
@@ -382,34 +444,40 @@ __device__ __forceinline__ void wave_store(const Cx<T> *v, Cx<T> *buf, int lane)
     }
 }
 
-// Passes 1..3 on data already in registers as pass-1 input.  On return the
-// lane holds output points j + r M/R3 (j = lane + 64 b) in v[b R3 + r].
+// Passes 1 and 2 on data in registers (v[b R1 + r] = point lane + 64 b +
+// r M/R1), up to the inputs of pass 3.
 template <typename T, int M, bool INV, typename W>
-__device__ __forceinline__ void wave_fft_regs(Cx<T> *v, Cx<T> *buf, int lane, const W &tw)
+__device__ __forceinline__ void wave_passes12(Cx<T> *v, Cx<T> *buf, int lane, const W &tw)
 {
     using P = WavePlan<M>;
-    wave_butterflies<T, M, P::R1, INV, false>(v, nullptr, 0);
+    wave_butterflies<T, M, P::R1, INV, false>(v, nullptr);
     wave_store<T, M, P::R1, 1>(v, buf, lane);
     wave_lds_sync();
     wave_load<T, M, P::R2>(v, buf, lane);
-    wave_butterflies<T, M, P::R2, INV, true>(v, tw.w2, 0);
+    wave_butterflies<T, M, P::R2, INV, true>(v, tw.w2);
     wave_lds_sync();
     wave_store<T, M, P::R2, P::R1>(v, buf, lane);
     wave_lds_sync();
     wave_load<T, M, P::R3>(v, buf, lane);
+    wave_lds_sync();
+}
+
+// Forward transform of registers in pass-1 layout; on return v[b R3 + r] is
+// point lane + 64 b + r M/R3.  Its plain pass-3 twiddles are looked up (one
+// forward transform per block).
+template <typename T, int M, typename W>
+__device__ __forceinline__ void wave_forward(Cx<T> *v, Cx<T> *buf, int lane, const W &w, const Twiddle<T> &tw)
+{
+    using P = WavePlan<M>;
+    wave_passes12<T, M, false>(v, buf, lane, w);
 #pragma unroll
     for (int b = 0; b < W::B3; ++b) {
-        Cx<T> w3[P::R3 - 1];
-        tw.pass3(lane, b, w3);
 #pragma unroll
         for (int r = 1; r < P::R3; ++r) {
-            Cx<T> t = w3[r - 1];
-            if (INV) { t.y = -t.y; }
-            v[b * P::R3 + r] = cmul(v[b * P::R3 + r], t);
+            v[b * P::R3 + r] = cmul(v[b * P::R3 + r], tw(4 * r * (lane + 64 * b)));
         }
-        mfcl::dftR<P::R3, INV>(&v[b * P::R3]);
+        mfcl::dftR<P::R3, false>(&v[b * P::R3]);
     }
-    wave_lds_sync();
 }
 
 // ---- half-size exchanges ------------------------------------------------
@@ -482,28 +550,15 @@ __device__ __forceinline__ void wave_exchange_half(Cx<T> *v, Cx<T> *buf, int lan
     for (int i = 0; i < Q; ++i) { v[i] = u[i]; }
 }
 
-// wave_fft_regs through a half buffer.
+// wave_passes12 through a half buffer.
 template <typename T, int M, bool INV, typename W>
-__device__ __forceinline__ void wave_fft_regs_half(Cx<T> *v, Cx<T> *buf, int lane, const W &tw)
+__device__ __forceinline__ void wave_passes12_half(Cx<T> *v, Cx<T> *buf, int lane, const W &tw)
 {
     using P = WavePlan<M>;
-    wave_butterflies<T, M, P::R1, INV, false>(v, nullptr, 0);
+    wave_butterflies<T, M, P::R1, INV, false>(v, nullptr);
     wave_exchange_half<T, M, P::R1, 1, P::R2>(v, buf, lane);
-    wave_butterflies<T, M, P::R2, INV, true>(v, tw.w2, 0);
+    wave_butterflies<T, M, P::R2, INV, true>(v, tw.w2);
     wave_exchange_half<T, M, P::R2, P::R1, P::R3>(v, buf, lane);
-#pragma unroll
-    for (int b = 0; b < W::B3; ++b) {
-        Cx<T> w3[P::R3 - 1];
-        tw.pass3(lane, b, w3);
-#pragma unroll
-        for (int r = 1; r < P::R3; ++r) {
-            Cx<T> t = w3[r - 1];
-            if (INV) { t.y = -t.y; }
-            v[b * P::R3 + r] = cmul(v[b * P::R3 + r], t);
-        }
-        mfcl::dftR<P::R3, INV>(&v[b * P::R3]);
-    }
-    wave_lds_sync();
 }
 
 // True when the Lt samples of the window at i are all equal (its exact

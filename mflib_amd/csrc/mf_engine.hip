@@ -4,7 +4,7 @@
 // one HIP stream, and after mf_initialize the device state:
 //   channels   [C][n_c]            samples in the handle precision
 //   templates  [rows][Lt]          FP64 demeaned unit-norm templates
-//   spectra    [rows][nfft/2+1]    conj(T^)/(2 nfft), handle precision
+//   spectra    [rows][nfft/2]      conj(T_k)/(nfft/2), handle precision
 //   rho        rows back to back   each row padded to a 64-sample multiple
 // plus the small descriptor tables the kernels read (lanes, rows, work
 // items) and the two-level twiddle tables of every FFT size in use.
@@ -21,6 +21,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <complex>
 #include <cstring>
 #include <map>
 #include <memory>
@@ -417,7 +418,7 @@ void initialize(mf_handle *h)
     for (int r = 0; r < nT; ++r) {
         auto &rp = h->rows[r];
         rp.specOff = specTotal;
-        specTotal += roundUp((1u << rp.logM) + 1, 32);
+        specTotal += static_cast<size_t>(1) << rp.logM;
         rp.tmplOff = tmplTotal;
         tmplTotal += roundUp(rp.Lt, 32);
     }
@@ -2591,6 +2592,36 @@ int mf_get_number_of_groups(const mf_handle *h, int *n)
     });
 }
 
+extern "C++" {
+namespace {
+
+// Forward FFT in place, z.size() a power of two: bit-reversed order, then
+// radix-2 stages.
+void transformPow2(std::vector<std::complex<double>> &z)
+{
+    const size_t n = z.size();
+    for (size_t i = 1, j = 0; i < n; ++i) {
+        size_t bit = n >> 1;
+        for (; (j & bit) != 0; bit >>= 1) { j ^= bit; }
+        j ^= bit;
+        if (i < j) { std::swap(z[i], z[j]); }
+    }
+    std::vector<std::complex<double>> w(n / 2);
+    for (size_t k = 0; k < n / 2; ++k) { w[k] = std::polar(1.0, -2.0 * M_PI * static_cast<double>(k) / n); }
+    for (size_t half = 1; half < n; half *= 2) {
+        for (size_t i = 0; i < n; i += 2 * half) {
+            for (size_t k = 0; k < half; ++k) {
+                const std::complex<double> t = w[k * (n / (2 * half))] * z[i + k + half];
+                z[i + k + half] = z[i + k] - t;
+                z[i + k] += t;
+            }
+        }
+    }
+}
+
+}  // namespace
+}  // extern "C++"
+
 int mf_template_spectrum(mf_handle *h, int row, void *outInterleaved, int cap, int *len)
 {
     return guard([&] {
@@ -2601,29 +2632,21 @@ int mf_template_spectrum(mf_handle *h, int row, void *outInterleaved, int cap, i
         const int N = 2 * M;
         if (len) { *len = M + 1; }
         if (outInterleaved == nullptr || cap < M + 1) { fail(MF_ERR_INVALID_ARGUMENT, "output buffer too small"); }
-        std::vector<char> raw((M + 1) * 2 * h->tsize);
-        MF_HIP(hipMemcpy(raw.data(), static_cast<const char *>(h->dSpec.p) + rp.specOff * 2 * h->tsize, raw.size(),
+        // the reversed template's spectrum from the FP64 taps: the kernels'
+        // own spectra are at other frequencies
+        std::vector<double> taps(rp.Lt);
+        MF_HIP(hipMemcpy(taps.data(), h->dTmpl.as<double>() + rp.tmplOff, taps.size() * sizeof(double),
                          hipMemcpyDeviceToHost));
-        // B[k] = exp(-2 pi i k (Lt-1)/N) * 2N * H[k]  (spectrum of the reversed template)
+        std::vector<std::complex<double>> z(N);
+        for (int m = 0; m < rp.Lt; ++m) { z[m] = taps[rp.Lt - 1 - m]; }
+        transformPow2(z);
         for (int k = 0; k <= M; ++k) {
-            double hr, hi;
             if (h->precision == MF_PRECISION_FLOAT) {
-                hr = reinterpret_cast<const float *>(raw.data())[2 * k];
-                hi = reinterpret_cast<const float *>(raw.data())[2 * k + 1];
+                static_cast<float *>(outInterleaved)[2 * k] = static_cast<float>(z[k].real());
+                static_cast<float *>(outInterleaved)[2 * k + 1] = static_cast<float>(z[k].imag());
             } else {
-                hr = reinterpret_cast<const double *>(raw.data())[2 * k];
-                hi = reinterpret_cast<const double *>(raw.data())[2 * k + 1];
-            }
-            const double ang = -2.0 * M_PI * static_cast<double>((static_cast<long long>(k) * (rp.Lt - 1)) % N) / N;
-            const double c = std::cos(ang), s = std::sin(ang);
-            const double br = 2.0 * N * (hr * c - hi * s);
-            const double bi = 2.0 * N * (hr * s + hi * c);
-            if (h->precision == MF_PRECISION_FLOAT) {
-                static_cast<float *>(outInterleaved)[2 * k] = static_cast<float>(br);
-                static_cast<float *>(outInterleaved)[2 * k + 1] = static_cast<float>(bi);
-            } else {
-                static_cast<double *>(outInterleaved)[2 * k] = br;
-                static_cast<double *>(outInterleaved)[2 * k + 1] = bi;
+                static_cast<double *>(outInterleaved)[2 * k] = z[k].real();
+                static_cast<double *>(outInterleaved)[2 * k + 1] = z[k].imag();
             }
         }
     });

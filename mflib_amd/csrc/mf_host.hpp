@@ -159,12 +159,12 @@ inline int referenceWindowLength(int nb, int nx, int *nfft, int *L)
     return 0;
 }
 
-// Two-level twiddle tables for W_{2M}: lo[i] = W^i (i < 64),
-// hi[j] = W^(64 j) (j < 2M/64), FP64 from cos/sin, rounded to T.
+// Two-level twiddle tables for W_{4M}: lo[i] = W^i (i < 64),
+// hi[j] = W^(64 j) (j < 4M/64), FP64 from cos/sin, rounded to T.
 template <typename T>
 std::vector<T> twiddleTable(int logM, bool high)
 {
-    const long long N = 2LL << logM;
+    const long long N = 4LL << logM;
     const int count = high ? static_cast<int>(N / 64) : 64;
     std::vector<T> v(2 * count);
     for (int i = 0; i < count; ++i) {

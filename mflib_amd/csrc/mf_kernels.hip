@@ -4,14 +4,14 @@
 //   lane; it serves every template row on that channel:
 //     1. load nfft samples (coalesced), FP64 block anchor (window mean),
 //        FP64 16-sample tile sums of (x-a) and (x-a)^2 via wave shuffles;
-//     2. forward real FFT of the anchored block (LDS Stockham), unpacked
-//        into X' = 2 X (kept in LDS for all rows);
+//     2. forward transform of the anchored block modulo z^M + i (see
+//        mf_device.hpp), kept in LDS for all rows;
 //     3. per template length: FP64 sliding window sums -> per-output
 //        scale sqrt(Lt)/sqrt(Lt*S2 - S1^2), with ill-conditioned windows
 //        flagged;
-//     4. per row: spectral product with the resident template spectrum
-//        (read from L2), inverse packing, inverse FFT, normalisation and
-//        the tooBig rule in the epilogue, one coalesced store of rho;
+//     4. per row: one complex product per bin with the resident template
+//        spectrum (read from L2), inverse FFT, normalisation and the tooBig
+//        rule in the epilogue, coalesced stores of rho;
 //        flagged windows are recomputed by an exact FP64 two-pass Pearson
 //        from the LDS copy of the samples.
 //   Blocks are overlap-save: block b covers outputs [bL, bL+L) and reads
@@ -327,7 +327,7 @@ __global__ __launch_bounds__(NT) void corr_kernel(const Item *__restrict__ items
     constexpr int LOGN = Log2<N>::value;
     static_assert(N % NT == 0, "block size");
     __shared__ T raw[N];
-    __shared__ Cx<T> Xs[M + 1];
+    __shared__ Cx<T> Xs[M];
     __shared__ Cx<T> Ws[M];
     __shared__ T sc[N];
     __shared__ double ts1[NTILE];
@@ -335,7 +335,7 @@ __global__ __launch_bounds__(NT) void corr_kernel(const Item *__restrict__ items
     __shared__ double tp1[NTILE + 1];
     __shared__ double tp2[NTILE + 1];
     __shared__ Cx<T> twlo[64];
-    __shared__ Cx<T> twhi[N / 64];
+    __shared__ Cx<T> twhi[N / 32];
     __shared__ double red[NT / 64];
 
     const Item item = items[blockIdx.x];
@@ -358,7 +358,7 @@ __global__ __launch_bounds__(NT) void corr_kernel(const Item *__restrict__ items
     }
 
     for (int i = tid; i < 64; i += NT) { twlo[i] = twloG[i]; }
-    for (int i = tid; i < N / 64; i += NT) { twhi[i] = twhiG[i]; }
+    for (int i = tid; i < N / 32; i += NT) { twhi[i] = twhiG[i]; }
     const Twiddle<T> tw{twlo, twhi};
 
     // 1. load the block, anchor, tile sums, energy
@@ -378,7 +378,6 @@ __global__ __launch_bounds__(NT) void corr_kernel(const Item *__restrict__ items
     const double a = block_sum<NT>(s, red) / nSamp;
     const T aT = static_cast<T>(a);
     double e = 0;
-    T *wf = reinterpret_cast<T *>(Ws);
 #pragma unroll
     for (int q = 0; q < SPT; ++q) {
         const int j = tid + q * NT;
@@ -395,23 +394,20 @@ __global__ __launch_bounds__(NT) void corr_kernel(const Item *__restrict__ items
             ts1[j >> 4] = t1;
             ts2[j >> 4] = t2;
         }
-        wf[j] = valid ? static_cast<T>(v[q] - aT) : T(0);
+        v[q] = valid ? static_cast<T>(v[q] - aT) : T(0);
     }
-    const double energy = block_sum<NT>(e, red);  // also publishes raw/ts/Ws
+    // u_j = (x_j - i x_{j+M}) W_{4M}^j: samples j and j + M are the thread's
+    // own q and q + SPT/2
+#pragma unroll
+    for (int q = 0; q < SPT / 2; ++q) {
+        const int j = tid + q * NT;
+        Xs[j] = cmul(Cx<T>{v[q], -v[q + SPT / 2]}, tw(j));
+    }
+    const double energy = block_sum<NT>(e, red);  // also publishes raw/ts/Xs
     tile_prefix<NTILE>(ts1, ts2, tp1, tp2, tid);   // read after the FFT's barriers
 
-    // 2. forward FFT of the packed block, unpack to X' = 2X
-    fft_lds<T, M, NT, false>(Ws, tw);
-    for (int k = tid; k <= M / 2; k += NT) {
-        const Cx<T> zk = Ws[k];
-        const Cx<T> zm = cconj(Ws[(M - k) & (M - 1)]);
-        const Cx<T> E = cadd(zk, zm);
-        const Cx<T> O = cmulmi(csub(zk, zm));
-        const Cx<T> WO = cmul(tw(k), O);
-        Xs[k] = cadd(E, WO);
-        Xs[M - k] = cconj(csub(E, WO));
-    }
-    __syncthreads();
+    // 2. forward transform of the block
+    fft_lds<T, M, NT, false>(Xs, tw);
 
     const double rmsBlk = sqrt(energy / nSamp);
     const double noise = kNoiseK / Eps<T>::rhoTol * Eps<T>::value * sqrt(static_cast<double>(LOGN)) *
@@ -430,30 +426,28 @@ __global__ __launch_bounds__(NT) void corr_kernel(const Item *__restrict__ items
             compute_scale<T, 16>(raw, ts1, ts2, tp1, tp2, sc, a, nValidSeg, Lt, noise, tid, NT);
             __syncthreads();
         }
-        // 4a. spectral product + inverse packing into Ws
+        // 4a. spectral product into Ws
         const Cx<T> *H = static_cast<const Cx<T> *>(row.H);
-        for (int k = tid; k <= M / 2; k += NT) {
-            const Cx<T> yk = cmul(Xs[k], H[k]);
-            const Cx<T> ym = cmul(Xs[M - k], H[M - k]);
-            const Cx<T> S = cadd(yk, cconj(ym));
-            const Cx<T> D = csub(yk, cconj(ym));
-            const Cx<T> P = cmul(cconj(tw(k)), D);
-            Ws[k] = cadd(S, cmuli(P));
-            if (k > 0) { Ws[M - k] = cadd(cconj(S), cmuli(cconj(P))); }
-        }
+        for (int k = tid; k < M; k += NT) { Ws[k] = cmul(Xs[k], H[k]); }
         __syncthreads();
-        // 4b. inverse FFT: Ws holds the correlation, interleaved = natural order
+        // 4b. inverse FFT; Ws[n] W_{4M}^-n = c_n - i c_{n+M}
         fft_lds<T, M, NT, true>(Ws, tw);
         // 4c. normalisation epilogue
         T *out = static_cast<T *>(row.out) + base;
-        const T *c = reinterpret_cast<const T *>(Ws);
-        for (int i = tid; i < nvRow; i += NT) {
-            const T f = sc[i];
-            if (f >= T(0)) {
-                T rho = c[i] * f;
-                if (fabs(rho) > T(1.1)) { rho = T(0); }
-                out[i] = rho;
+        const auto store = [&](int i, T c) {
+            if (i < nvRow) {
+                const T f = sc[i];
+                if (f >= T(0)) {
+                    T rho = c * f;
+                    if (fabs(rho) > T(1.1)) { rho = T(0); }
+                    out[i] = rho;
+                }
             }
+        };
+        for (int n = tid; n < M; n += NT) {
+            const Cx<T> c = cmul(Ws[n], cconj(tw(n)));
+            store(n, c.x);
+            store(n + M, -c.y);
         }
         // 4d. exact FP64 two-pass Pearson for flagged windows
         {
@@ -505,10 +499,10 @@ __global__ __launch_bounds__(NT) void corr_kernel(const Item *__restrict__ items
 // ---------------------------------------------------------------------------
 // corr2_kernel: same contract as corr_kernel, built from wave-level FFTs.
 // Wave 0 computes the forward FFT while waves 1-3 build the normalisation
-// scale; then every wave takes whole template rows (product with the
-// template spectrum straight into pass-1 registers, three register passes,
-// epilogue straight from pass-3 registers), so the row loop has no block
-// barrier.  Rows are processed in groups of equal template length; the
+// scale; then every wave takes whole template rows (one complex product per
+// bin in pass-1 registers, three register passes, epilogue straight from
+// pass-3 registers), so the row loop has no block barrier and a row's only
+// LDS traffic is the two exchanges between passes and the scale reads.  Rows are processed in groups of equal template length; the
 // scale of a group is shared by its rows.
 // ---------------------------------------------------------------------------
 
@@ -598,17 +592,6 @@ __device__ __forceinline__ void fixup_row_wave(const T *raw, const T *sc, gptr<c
     }
 }
 
-template <typename T>
-struct Vec2;
-template <>
-struct Vec2<float> {
-    using type = float2;
-};
-template <>
-struct Vec2<double> {
-    using type = double2;
-};
-
 // Shape of corr2_kernel<T, M>:
 //  - SHARED: a block-wide scale buffer for groups of rows of one template
 //    length (FP32 up to M = 1024, FP64 up to M = 512);
@@ -645,9 +628,6 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
     constexpr int SPT = N / NT;
     constexpr int LOGN = Log2<N>::value;
     constexpr int Q = M / 64;
-    // (k, M-k) pair steps per lane for k < M/2; the self-paired bin k = M/2
-    // has a closed form (its twiddle is exactly -i) and is done apart
-    constexpr int KP = M / 2 / 64;
     constexpr int NWAVE = NT / 64;
     constexpr int XH = XHalf<M>::size;
     constexpr int XW = HALF ? XH : XBuf<M>::size;  // exchange buffer of one wave
@@ -655,11 +635,10 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
     static_assert(N % NT == 0 && NWAVE == 4, "block shape");
     static_assert(2 * XH == XBuf<M>::size, "two half buffers make one full buffer");
     __shared__ T raw[N];
-    __shared__ Cx<T> Xs[M + 1];
+    __shared__ Cx<T> Xs[M];
     __shared__ __align__(16) T sc[SHARED ? N : 1];
     // one exchange buffer per wave (half size with HALF; then the first two
-    // together are the full buffer of the forward transform and of the
-    // packed input)
+    // together are the full buffer of the forward transform)
     __shared__ Cx<T> xb[NWAVE * XW];
     // FP64 tile prefix sums; FP64 correlation also keeps the tile sums (FP32
     // builds the prefix in place over the sums)
@@ -668,7 +647,7 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
     __shared__ double tsd1[sizeof(T) == 8 ? NTILE : 1];
     __shared__ double tsd2[sizeof(T) == 8 ? NTILE : 1];
     __shared__ Cx<T> twlo[64];
-    __shared__ Cx<T> twhi[N / 64];
+    __shared__ Cx<T> twhi[N / 32];
     __shared__ double red[NWAVE];
     double *ts1 = sizeof(T) == 8 ? tsd1 : tp1;
     double *ts2 = sizeof(T) == 8 ? tsd2 : tp2;
@@ -694,10 +673,10 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
         return;
     }
     for (int i = tid; i < 64; i += NT) { twlo[i] = twloG[i]; }
-    for (int i = tid; i < N / 64; i += NT) { twhi[i] = twhiG[i]; }
+    for (int i = tid; i < N / 32; i += NT) { twhi[i] = twhiG[i]; }
     const Twiddle<T> tw{twlo, twhi};
 
-    // A. load, anchor, tile sums, energy; packed anchored input -> xb (full)
+    // A. load, anchor, tile sums, energy
     const gptr<const T> x = to_global(static_cast<const T *>(sg.x));
     const int nSamp = static_cast<int>(min(static_cast<long long>(N), sg.n - base));
     T v0[SPT];
@@ -713,7 +692,6 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
     const double a = uniform(block_sum<NT>(s, red) / nSamp);  // scalar registers: used by every row
     const T aT = static_cast<T>(a);
     double e = 0;
-    T *xin = reinterpret_cast<T *>(xb);
 #pragma unroll
     for (int q = 0; q < SPT; ++q) {
         const int j = tid + q * NT;
@@ -730,7 +708,6 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
             ts1[j / TILE] = t1;
             ts2[j / TILE] = t2;
         }
-        xin[2 * xpad(j >> 1) + (j & 1)] = valid ? static_cast<T>(v0[q] - aT) : T(0);
     }
     const double energy = block_sum<NT>(e, red);
     tile_prefix<NTILE>(ts1, ts2, tp1, tp2, tid);  // in place for FP32 (each lane reads its tiles first)
@@ -739,49 +716,30 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
     const double noise = uniform(kNoiseK / Eps<T>::rhoTol * Eps<T>::value * sqrt(static_cast<double>(LOGN)) *
                                  static_cast<double>(sg.hmax) * rmsBlk);
     WaveTwiddles<T, M, !HALF> wt;
-    wt.init(lane, tw);
+    wt.initPass2(lane, tw);
     Cx<T> v[Q];
 
-    // B. forward FFT + unpack into Xs (wave 0, full buffer)
+    // B. forward transform of u_j = (x_j - i x_{j+M}) W_{4M}^j into Xs (wave
+    // 0, full buffer); the lane's points are lane + 64 q
     auto forwardFft = [&]() {
-        Cx<T> *buf = xb;
-        wave_load<T, M, P::R1>(v, buf, lane);
-        wave_lds_sync();
-        wave_fft_regs<T, M, false>(v, buf, lane, wt);
-        // natural-order store of pass 3 (point j + r M/R3, j = lane + 64 b)
-        constexpr int B3 = M / (P::R3 * 64);
-        Cx<T> *po = buf + xpad(lane);
+        const auto sample = [&](int j) { return j < nSamp ? static_cast<T>(raw[j] - aT) : T(0); };
 #pragma unroll
-        for (int b = 0; b < B3; ++b) {
+        for (int q = 0; q < Q; ++q) {
+            const int j = lane + 64 * q;
+            // pass-1 register of point j = lane + 64 b + r M/R1
+            const int reg = (q % (Q / P::R1)) * P::R1 + q / (Q / P::R1);
+            v[reg] = cmul(Cx<T>{sample(j), -sample(j + M)}, tw(j));
+        }
+        wave_forward<T, M>(v, xb, lane, wt, tw);
 #pragma unroll
-            for (int r = 0; r < P::R3; ++r) { po[cpad(64 * b + r * (M / P::R3))] = v[b * P::R3 + r]; }
-        }
-        wave_lds_sync();
-        // unpack pairs (k, M-k), k = lane + 64 t < M/2
-        const Cx<T> *pm = buf + xpad(M - lane);
-        const Cx<T> wlo = twlo[lane];
+        for (int b = 0; b < Q / P::R3; ++b) {
 #pragma unroll
-        for (int t = 0; t < KP; ++t) {
-            const int k = lane + 64 * t;
-            const Cx<T> zk = po[68 * t];
-            const Cx<T> zm = cconj(k == 0 ? po[0] : pm[-68 * t]);
-            const Cx<T> E = cadd(zk, zm);
-            const Cx<T> O = cmulmi(csub(zk, zm));
-            const Cx<T> WO = cmul(cmul(wlo, twhi[t]), O);
-            Xs[k] = cadd(E, WO);
-            Xs[M - k] = cconj(csub(E, WO));
+            for (int r = 0; r < P::R3; ++r) { Xs[lane + 64 * b + r * (M / P::R3)] = v[b * P::R3 + r]; }
         }
-        // k = M/2: E = 2 Re z, O = 2 Im z, twiddle -i, so X' = 2 conj(z)
-        if (lane == 0) {
-            const Cx<T> z = buf[xpad(M / 2)];
-            Xs[M / 2] = Cx<T>{z.x + z.x, -(z.y + z.y)};
-        }
-        wave_lds_sync();
     };
 
     // C. one template row on this wave, in two halves.  startRow: spectral
-    // product + inverse packing and the three register passes (the result
-    // stays in v).  finishRow: the row's scale when it has no shared one,
+    // product and the three register passes (the result stays in v).  finishRow: the row's scale when it has no shared one,
     // then the normalisation epilogue straight from the pass-3 registers.
     // A wave's row sequence runs start(r0), then for each next row r:
     // finish(previous), start(r), and finally finish(last).  start(r)
@@ -789,17 +747,11 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
     // the load is in flight through r's transform and epilogue; the
     // epilogue issues the same (range-checked) stores on every path, so
     // the wait for that spectrum never waits for those stores.
-    Cx<T> hk[KP], hm[KP];  // template spectrum pairs (H[k], H[M-k]), k < M/2
-    Cx<T> hmid;            // H[M/2]
+    Cx<T> hk[Q];  // template spectrum at the lane's points lane + 64 q
     auto loadH = [&](const void *Hp) {
         const gptr<const Cx<T>> H = to_global(static_cast<const Cx<T> *>(Hp));
 #pragma unroll
-        for (int t = 0; t < KP; ++t) {
-            const int k = lane + 64 * t;
-            hk[t] = load_cx(H, k);
-            hm[t] = load_cx(H, M - k);
-        }
-        hmid = load_cx(H, M / 2);
+        for (int q = 0; q < Q; ++q) { hk[q] = load_cx(H, lane + 64 * q); }
     };
     auto rowValid = [&](const Row &row) {
         return static_cast<int>(max(0ll, min(static_cast<long long>(sg.L), row.nOut - base)));
@@ -812,115 +764,47 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
         }
         if (!PREFETCH) { loadH(row.H); }
         Cx<T> *buf = xb + wave * XW;
-        if constexpr (!HALF) {
-            // (k, M-k) pair per lane step (k = lane + 64 t; tw(k) = lo[lane] hi[t])
-            const Cx<T> wlo = twlo[lane];
-            Cx<T> *pk = buf + xpad(lane);
-            Cx<T> *pm = buf + xpad(M - lane);
 #pragma unroll
-            for (int t = 0; t < KP; ++t) {
-                const int k = lane + 64 * t;
-                const Cx<T> yk = cmul(Xs[k], hk[t]);
-                const Cx<T> ym = cmul(Xs[M - k], hm[t]);
-                const Cx<T> S = cadd(yk, cconj(ym));
-                const Cx<T> D = csub(yk, cconj(ym));
-                const Cx<T> Pp = cmul(cconj(cmul(wlo, twhi[t])), D);
-                pk[68 * t] = cadd(S, cmuli(Pp));
-                if (k > 0) { pm[-68 * t] = cadd(cconj(S), cmuli(cconj(Pp))); }
-            }
-            // k = M/2 (y = X H): S = 2 Re y, D = 2i Im y, twiddle -i, so Z = 2 conj(y)
-            if (lane == 0) {
-                const Cx<T> y = cmul(Xs[M / 2], hmid);
-                buf[xpad(M / 2)] = Cx<T>{y.x + y.x, -(y.y + y.y)};
-            }
-            // the next row's spectrum is in flight through this row's
-            // transform and epilogue
-            loadH(nextH);
-            wave_lds_sync();
-            wave_load<T, M, P::R1>(v, buf, lane);
-            wave_lds_sync();
-            wave_fft_regs<T, M, true>(v, buf, lane, wt);
-            return;
+        for (int q = 0; q < Q; ++q) {
+            const int reg = (q % (Q / P::R1)) * P::R1 + q / (Q / P::R1);
+            v[reg] = cmul(Xs[lane + 64 * q], hk[q]);
         }
-        // (k, M-k) pair per lane step (k = lane + 64 t; tw(k) = lo[lane] hi[t]).
-        // Points k < M/2 are the first half of the pass-1 input, M - k and
-        // M/2 the second: the first half goes out and comes back in while
-        // the second waits in registers.
-        const Cx<T> wlo = twlo[lane];
-        Cx<T> *pk = buf + xpad(lane);
-        Cx<T> *pm = buf - cpad(M / 2) + xpad(M - lane);
-        Cx<T> zm[KP];
-#pragma unroll
-        for (int t = 0; t < KP; ++t) {
-            const int k = lane + 64 * t;
-            const Cx<T> yk = cmul(Xs[k], hk[t]);
-            const Cx<T> ym = cmul(Xs[M - k], hm[t]);
-            const Cx<T> S = cadd(yk, cconj(ym));
-            const Cx<T> D = csub(yk, cconj(ym));
-            const Cx<T> Pp = cmul(cconj(cmul(wlo, twhi[t])), D);
-            pk[68 * t] = cadd(S, cmuli(Pp));
-            zm[t] = cadd(cconj(S), cmuli(cconj(Pp)));
+        // the next row's spectrum is in flight through this row's transform
+        // and epilogue
+        if (PREFETCH) { loadH(nextH); }
+        if constexpr (HALF) {
+            wave_passes12_half<T, M, true>(v, buf, lane, wt);
+        } else {
+            wave_passes12<T, M, true>(v, buf, lane, wt);
         }
-        // k = M/2 (y = X H): S = 2 Re y, D = 2i Im y, twiddle -i, so Z = 2 conj(y)
-        const Cx<T> ymid = cmul(Xs[M / 2], hmid);
-        wave_lds_sync();
-        wave_load_half<T, M, P::R1, 0>(v, buf, lane);
-        wave_lds_sync();
-#pragma unroll
-        for (int t = 0; t < KP; ++t) {
-            if (lane + 64 * t > 0) { pm[-68 * t] = zm[t]; }
-        }
-        if (lane == 0) { buf[0] = Cx<T>{ymid.x + ymid.x, -(ymid.y + ymid.y)}; }  // point M/2 of half 1
-        wave_lds_sync();
-        wave_load_half<T, M, P::R1, 1>(v, buf, lane);
-        wave_lds_sync();
-        wave_fft_regs_half<T, M, true>(v, buf, lane, wt);
+        wave_pass3_inverse<T, M>(v, wt);
     };
-    // rho = c * scale for the pass-3 outputs in half H of the block (the
-    // lane's points j + r M/R3 with r in [H R3/2, (H+1) R3/2): outputs
-    // [H N/2, (H+1) N/2)), paired stores; scl[i - first] is output i's
+    // rho = c * scale for the outputs of half H of the block, [H M, (H+1) M):
+    // the real parts (H = 0) or the negated imaginary parts (H = 1) of the
+    // lane's points n = lane + 64 b + r M/R3; scl[i - first] is output i's
     // scale.  Flagged windows (scale -1) are overwritten by the exact
     // fix-up; for the others |rho| <= 1 + O(eps), so the reference's tooBig
     // rule (|rho| > 1.1 -> 0) cannot fire and is not evaluated.  The scale
     // reads stay inside the scale buffer for every position.  The store
-    // resource ends at the last whole pair of valid outputs, so invalid
-    // pairs are dropped; an odd last output is stored apart.
-    using V2 = typename Vec2<T>::type;
+    // resource ends at the last valid output, so invalid stores are dropped.
     constexpr int B3 = M / (P::R3 * 64);
     auto epilogueHalf = [&](auto hTag, const T *scl, int first, T *outRow, int nvRow) {
         constexpr int H = decltype(hTag)::value;
-        constexpr int R0 = H * (P::R3 / 2), R1e = (H + 1) * (P::R3 / 2);
-        constexpr int NQH = B3 * (P::R3 / 2);
-        const __amdgpu_buffer_rsrc_t rs = buffer_rsrc(outRow, static_cast<int>(sizeof(T)) * (nvRow & ~1));
-        const T *sp = scl - first + 2 * lane;
-        V2 f[NQH];
+        const __amdgpu_buffer_rsrc_t rs = buffer_rsrc(outRow, static_cast<int>(sizeof(T)) * nvRow);
+        const T *sp = scl - first + H * M + lane;
+        T f[Q];
 #pragma unroll
         for (int b = 0; b < B3; ++b) {
 #pragma unroll
-            for (int r = R0; r < R1e; ++r) {
-                f[b * (P::R3 / 2) + r - R0] = *reinterpret_cast<const V2 *>(sp + 2 * (64 * b + r * (M / P::R3)));
-            }
+            for (int r = 0; r < P::R3; ++r) { f[b * P::R3 + r] = sp[64 * b + r * (M / P::R3)]; }
         }
 #pragma unroll
         for (int b = 0; b < B3; ++b) {
 #pragma unroll
-            for (int r = R0; r < R1e; ++r) {
+            for (int r = 0; r < P::R3; ++r) {
                 const int q = b * P::R3 + r;
-                const V2 fq = f[b * (P::R3 / 2) + r - R0];
-                const int i0 = 2 * lane + 2 * (64 * b + r * (M / P::R3));
-                buffer_store_pair(v[q].x * fq.x, v[q].y * fq.y, rs, static_cast<int>(sizeof(T)) * i0);
-            }
-        }
-        if (nvRow & 1) {
-            gptr<T> outG = to_global(outRow);
-#pragma unroll
-            for (int b = 0; b < B3; ++b) {
-#pragma unroll
-                for (int r = R0; r < R1e; ++r) {
-                    const int q = b * P::R3 + r;
-                    const int i0 = 2 * lane + 2 * (64 * b + r * (M / P::R3));
-                    if (i0 == nvRow - 1) { outG[i0] = v[q].x * f[b * (P::R3 / 2) + r - R0].x; }
-                }
+                const int i = H * M + lane + 64 * b + r * (M / P::R3);
+                buffer_store(H == 0 ? v[q].x * f[q] : v[q].y * -f[q], rs, static_cast<int>(sizeof(T)) * i);
             }
         }
     };
@@ -1041,26 +925,32 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
     // the block; rows of smaller groups (every row without the buffer) are
     // "solo": each wave takes every NWAVE-th of them and computes its row's
     // scale itself, so no wave waits for a group it has no row in.
-    bool fftDone = false;
+    auto groupEnd = [&](int g0) {
+        int g1 = g0 + 1;
+        while (g1 < rowEnd && rows[g1].Lt == rows[g0].Lt) { ++g1; }
+        return g1;
+    };
+    // wave 0 transforms while waves 1..3 build the first group's scale, if
+    // it is a shared one
+    const bool firstShared = SHARED && groupEnd(sg.rowBegin) - sg.rowBegin >= kCorr2SharedGroup;
+    int myFlags = 0;
+    if (wave == 0) {
+        forwardFft();
+    } else if (firstShared) {
+        myFlags = compute_scale<T, TILE, 1, QUEUE>(raw, ts1, ts2, tp1, tp2, sc, a, nValidSeg, rows[sg.rowBegin].Lt,
+                                                   noise, tid - 64, NT - 64);
+    }
+    // pass-3 twiddles only now: the forward transform is over, and so is its
+    // need of registers
+    wt.initPass3(lane, tw);
+    if (!firstShared) { __syncthreads(); }
     if constexpr (SHARED) {
         for (int g0 = sg.rowBegin; g0 < rowEnd;) {
-            const int Lt = rows[g0].Lt;
-            int g1 = g0 + 1;
-            while (g1 < rowEnd && rows[g1].Lt == Lt) { ++g1; }
+            const int g1 = groupEnd(g0);
             if (g1 - g0 >= kCorr2SharedGroup) {
-                int myFlags = 0;
-                if (!fftDone) {
-                    // wave 0 transforms while waves 1..3 build the scale
-                    if (wave == 0) {
-                        forwardFft();
-                    } else {
-                        myFlags = compute_scale<T, TILE, 1, QUEUE>(raw, ts1, ts2, tp1, tp2, sc, a, nValidSeg, Lt, noise,
-                                                         tid - 64, NT - 64);
-                    }
-                    fftDone = true;
-                } else {
-                    myFlags = compute_scale<T, TILE, 1, QUEUE>(raw, ts1, ts2, tp1, tp2, sc, a, nValidSeg, Lt, noise, tid,
-                                                               NT);
+                if (g0 != sg.rowBegin) {
+                    myFlags = compute_scale<T, TILE, 1, QUEUE>(raw, ts1, ts2, tp1, tp2, sc, a, nValidSeg, rows[g0].Lt,
+                                                               noise, tid, NT);
                 }
                 const double flagSum = uniform(block_sum<NT>(static_cast<double>(myFlags), red));  // scalar registers
                 const bool anyFlag = flagSum > 0.0;
@@ -1079,10 +969,6 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
             }
             g0 = g1;
         }
-    }
-    if (!fftDone) {
-        if (wave == 0) { forwardFft(); }
-        __syncthreads();
     }
     // Solo rows of this wave in order: the k-th solo row of the segment
     // belongs to wave k mod NWAVE.  nextSolo walks the groups (scalar
@@ -1119,7 +1005,9 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
     }
 }
 
-// Template demean / unit-norm (FP64) and spectrum conj(T^)/(2 nfft).
+// Template demean / unit-norm (FP64) and its spectrum H_k = conj(T_k)/M at the
+// roots the correlation kernels use (T the M-point transform of
+// (t_j - i t_{j+M}) W_{4M}^j).
 template <int M>
 __global__ __launch_bounds__(NT) void tmpl_kernel(const TmplJob *__restrict__ jobs, int precision,
                                                   const Cx<double> *__restrict__ twloG,
@@ -1128,12 +1016,12 @@ __global__ __launch_bounds__(NT) void tmpl_kernel(const TmplJob *__restrict__ jo
     constexpr int N = 2 * M;
     __shared__ Cx<double> Z[M];
     __shared__ Cx<double> twlo[64];
-    __shared__ Cx<double> twhi[N / 64];
+    __shared__ Cx<double> twhi[N / 32];
     __shared__ double red[NT / 64];
     const TmplJob job = jobs[blockIdx.x];
     const int tid = threadIdx.x;
     for (int i = tid; i < 64; i += NT) { twlo[i] = twloG[i]; }
-    for (int i = tid; i < N / 64; i += NT) { twhi[i] = twhiG[i]; }
+    for (int i = tid; i < N / 32; i += NT) { twhi[i] = twhiG[i]; }
     const Twiddle<double> tw{twlo, twhi};
     double s = 0;
     for (int m = tid; m < job.Lt; m += NT) { s += job.t[m]; }
@@ -1145,40 +1033,21 @@ __global__ __launch_bounds__(NT) void tmpl_kernel(const TmplJob *__restrict__ jo
     }
     const double norm = sqrt(block_sum<NT>(e, red));
     const double scale = norm > 0 ? 1.0 / norm : 0.0;
-    double *zf = reinterpret_cast<double *>(Z);
-    for (int m = tid; m < N; m += NT) {
-        double tv = 0;
-        if (m < job.Lt) {
-            tv = (job.t[m] - mean) * scale;
-            job.tOut[m] = tv;
-        }
-        zf[m] = tv;
-    }
+    const auto tap = [&](int m) { return m < job.Lt ? (job.t[m] - mean) * scale : 0.0; };
+    for (int m = tid; m < job.Lt; m += NT) { job.tOut[m] = tap(m); }
+    for (int j = tid; j < M; j += NT) { Z[j] = cmul(Cx<double>{tap(j), -tap(j + M)}, tw(j)); }
     __syncthreads();
     fft_lds<double, M, NT, false>(Z, tw);
-    const double hs = 1.0 / (2.0 * N);
+    constexpr double hs = 1.0 / M;
     double hmax = 0;
-    for (int k = tid; k <= M / 2; k += NT) {
-        const Cx<double> zk = Z[k];
-        const Cx<double> zm = cconj(Z[(M - k) & (M - 1)]);
-        const Cx<double> E = cadd(zk, zm);
-        const Cx<double> O = cmulmi(csub(zk, zm));
-        const Cx<double> WO = cmul(tw(k), O);
-        const Cx<double> tk = cadd(E, WO);             // 2 T^[k]
-        const Cx<double> tm = cconj(csub(E, WO));      // 2 T^[M-k]
-        hmax = fmax(hmax, 0.5 * sqrt(tk.x * tk.x + tk.y * tk.y));
-        hmax = fmax(hmax, 0.5 * sqrt(tm.x * tm.x + tm.y * tm.y));
-        // conj(T^)/(2N) = conj(2 T^) / (4N)
-        const Cx<double> hk{tk.x * hs * 0.5, -tk.y * hs * 0.5};
-        const Cx<double> hm{tm.x * hs * 0.5, -tm.y * hs * 0.5};
+    for (int k = tid; k < M; k += NT) {
+        const Cx<double> z = Z[k];
+        hmax = fmax(hmax, sqrt(z.x * z.x + z.y * z.y));
         if (precision == 0) {
-            Cx<float> *H = static_cast<Cx<float> *>(job.H);
-            H[k] = Cx<float>{static_cast<float>(hk.x), static_cast<float>(hk.y)};
-            H[M - k] = Cx<float>{static_cast<float>(hm.x), static_cast<float>(hm.y)};
+            static_cast<Cx<float> *>(job.H)[k] =
+                Cx<float>{static_cast<float>(z.x * hs), static_cast<float>(-z.y * hs)};
         } else {
-            Cx<double> *H = static_cast<Cx<double> *>(job.H);
-            H[k] = hk;
-            H[M - k] = hm;
+            static_cast<Cx<double> *>(job.H)[k] = Cx<double>{z.x * hs, -z.y * hs};
         }
     }
     hmax = block_max<NT>(hmax, red);

@@ -40,7 +40,7 @@ constexpr int kCorr2SharedGroup = 4;
 
 // One template row.
 struct Row {
-    const void *H;        // conj(spectrum)/(2 nfft), nfft/2+1 complex
+    const void *H;        // template spectrum H_k = conj(T_k)/M, M = nfft/2 complex
     const double *tmpl;   // demeaned unit-norm template (FP64), Lt samples
     void *out;            // correlation output row
     int nOut;             // outputs of this row

@@ -2,7 +2,7 @@
 //
 // HBM layout:
 //   library   per add call: FP64 raw and prepared templates [n][Lt], and
-//             one spectrum per supported FFT size [n][logM][nfft/2+1]
+//             one spectrum per supported FFT size [n][logM][nfft/2]
 //   arena     one allocation of the budget, carved per request into
 //             [inputs copied from host][rho rows (template, channel)]
 //   slots     per in-flight batch: descriptor tables and dead-trace partials
@@ -387,7 +387,7 @@ void addTemplates(mf_server *s, int n, const int *lengths, const double *const *
         for (int lg = mfk::kMinLogM; lg <= hiLog; ++lg) {
             if ((2LL << lg) - lengths[i] + 1 < 2) { continue; }
             sOff[i][lg] = specTotal;
-            specTotal += roundUp((1u << lg) + 1, 32);
+            specTotal += static_cast<size_t>(1) << lg;
         }
     }
     auto chunk = std::make_unique<LibChunk>();

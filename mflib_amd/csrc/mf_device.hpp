@@ -198,6 +198,49 @@ __device__ __forceinline__ float uniform(float v)
     return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
 }
 
+// ---- wave scans on DPP moves ---------------------------------------------
+// v of the lane CTRL names (0 where it names none, or in rows outside
+// ROWS); no LDS permute, so a step costs a few cycles instead of an LDS
+// round trip.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_move(int v)
+{
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_move(float v)
+{
+    return __int_as_float(dpp_move<CTRL, ROWS>(__float_as_int(v)));
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_move(double v)
+{
+    return __hiloint2double(dpp_move<CTRL, ROWS>(__double2hiint(v)), dpp_move<CTRL, ROWS>(__double2loint(v)));
+}
+// Inclusive sum over the lanes 0..lane of the wave: shifts by 1, 2, 4, 8
+// inside rows of 16, then lane 15 of each row to the next row and lane 31 to
+// the upper half.
+template <typename T>
+__device__ __forceinline__ T wave_scan_sum(T v)
+{
+    v += dpp_move<0x111, 0xf>(v);
+    v += dpp_move<0x112, 0xf>(v);
+    v += dpp_move<0x114, 0xf>(v);
+    v += dpp_move<0x118, 0xf>(v);
+    v += dpp_move<0x142, 0xa>(v);
+    v += dpp_move<0x143, 0xc>(v);
+    return v;
+}
+__device__ __forceinline__ float read_lane(float v, int l)
+{
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ __forceinline__ double read_lane(double v, int l)
+{
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                            __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+
 // ---- block reductions -------------------------------------------------
 __device__ __forceinline__ double wave_sum(double v)
 {
@@ -334,26 +377,42 @@ constexpr double turnSin(int num, int den) { return turnCos(4 * num - den, 4 * d
 //           the transform's own twiddle W_M^-(j r) and the lane part of the
 //           output weight W_{4M}^-n, n = j + m M/R3.  What is left of that
 //           weight, W_{4 R3}^-m, is the same for every lane (unweight3).
+// W2LDS: the pass-2 rows come from a table in LDS ((R2 - 1) R1 entries, a
+// block's own; each read is a broadcast of R1 consecutive entries) instead of
+// 2 (R2 - 1) registers.
 // W3REG: a pass-3 row per butterfly in registers; otherwise one row for
 // butterfly 0 and a constant complex product per element for the others
 // (no LDS reads, and 2 (B3 - 1) R3 fewer registers).
-template <typename T, int M, bool W3REG = true>
+template <typename T, int M, bool W2LDS, bool W3REG>
 struct WaveTwiddles {
     using P = WavePlan<M>;
     static constexpr int NS2 = P::R1;
     static constexpr int B3 = M / (P::R3 * 64);
     static constexpr int W3 = W3REG ? B3 : 1;
-    Cx<T> w2[P::R2 - 1];
+    static constexpr int TABLE = W2LDS ? (P::R2 - 1) * P::R1 : 1;
+    Cx<T> w2reg[W2LDS ? 1 : P::R2 - 1];
     Cx<T> w3[W3][P::R3];
-    __device__ __forceinline__ void initPass2(int lane, const Twiddle<T> &tw)
+    const Cx<T> *w2p;  // LDS, at the lane's entry of the first row
+    // Row r of pass 2 (r = 1 .. R2 - 1).
+    __device__ __forceinline__ Cx<T> w2(int r) const { return W2LDS ? w2p[(r - 1) * P::R1] : w2reg[r - 1]; }
+    // The block's pass-2 table (the caller synchronises).
+    __device__ __forceinline__ static void fill(Cx<T> *table, int tid, int threads, const Twiddle<T> &tw)
+    {
+        if constexpr (W2LDS) {
+            for (int i = tid; i < TABLE; i += threads) {
+                table[i] = cconj(tw((4 * M / (NS2 * P::R2)) * (i / P::R1 + 1) * (i % P::R1)));
+            }
+        }
+    }
+    __device__ __forceinline__ void init(int lane, const Twiddle<T> &tw, const Cx<T> *table)
     {
         const int k2 = lane & (NS2 - 1);
-        const int s2 = (4 * M / (NS2 * P::R2)) * k2;
+        w2p = table + k2;
+        if constexpr (!W2LDS) {
+            const int s2 = (4 * M / (NS2 * P::R2)) * k2;
 #pragma unroll
-        for (int r = 1; r < P::R2; ++r) { w2[r - 1] = cconj(tw(r * s2)); }
-    }
-    __device__ __forceinline__ void initPass3(int lane, const Twiddle<T> &tw)
-    {
+            for (int r = 1; r < P::R2; ++r) { w2reg[r - 1] = cconj(tw(r * s2)); }
+        }
 #pragma unroll
         for (int b = 0; b < W3; ++b) {
 #pragma unroll
@@ -407,25 +466,26 @@ __device__ __forceinline__ void wave_pass3_inverse(Cx<T> *v, const W &tw)
     unweight3<1, T, M>(v);
 }
 
-// Butterflies of one pass; with TWIDDLE, element r of each is first
-// multiplied by w[r-1] (a row of inverse twiddles, conjugated for forward
-// transforms).
-template <typename T, int M, int R, bool INV, bool TWIDDLE>
-__device__ __forceinline__ void wave_butterflies(Cx<T> *v, const Cx<T> *w)
+// Inverse butterflies of pass 1, and of pass 2 with their twiddles.
+template <typename T, int M>
+__device__ __forceinline__ void wave_pass1(Cx<T> *v)
 {
-    constexpr int B = M / (R * 64);
+    constexpr int R = WavePlan<M>::R1;
 #pragma unroll
-    for (int b = 0; b < B; ++b) {
-        if constexpr (TWIDDLE) {
+    for (int b = 0; b < M / (R * 64); ++b) { mfcl::dftR<R, true>(&v[b * R]); }
+}
+template <typename T, int M, typename W>
+__device__ __forceinline__ void wave_pass2(Cx<T> *v, const W &tw)
+{
+    constexpr int R = WavePlan<M>::R2, B = M / (R * 64);
 #pragma unroll
-            for (int r = 1; r < R; ++r) {
-                Cx<T> t = w[r - 1];
-                if (!INV) { t.y = -t.y; }
-                v[b * R + r] = cmul(v[b * R + r], t);
-            }
-        }
-        mfcl::dftR<R, INV>(&v[b * R]);
+    for (int r = 1; r < R; ++r) {
+        const Cx<T> w = tw.w2(r);
+#pragma unroll
+        for (int b = 0; b < B; ++b) { v[b * R + r] = cmul(v[b * R + r], w); }
     }
+#pragma unroll
+    for (int b = 0; b < B; ++b) { mfcl::dftR<R, true>(&v[b * R]); }
 }
 
 template <typename T, int M, int R, int NS>
@@ -444,17 +504,17 @@ __device__ __forceinline__ void wave_store(const Cx<T> *v, Cx<T> *buf, int lane)
     }
 }
 
-// Passes 1 and 2 on data in registers (v[b R1 + r] = point lane + 64 b +
-// r M/R1), up to the inputs of pass 3.
-template <typename T, int M, bool INV, typename W>
+// Inverse passes 1 and 2 on data in registers (v[b R1 + r] = point lane +
+// 64 b + r M/R1), up to the inputs of pass 3.
+template <typename T, int M, typename W>
 __device__ __forceinline__ void wave_passes12(Cx<T> *v, Cx<T> *buf, int lane, const W &tw)
 {
     using P = WavePlan<M>;
-    wave_butterflies<T, M, P::R1, INV, false>(v, nullptr);
+    wave_pass1<T, M>(v);
     wave_store<T, M, P::R1, 1>(v, buf, lane);
     wave_lds_sync();
     wave_load<T, M, P::R2>(v, buf, lane);
-    wave_butterflies<T, M, P::R2, INV, true>(v, tw.w2);
+    wave_pass2<T, M>(v, tw);
     wave_lds_sync();
     wave_store<T, M, P::R2, P::R1>(v, buf, lane);
     wave_lds_sync();
@@ -462,22 +522,68 @@ __device__ __forceinline__ void wave_passes12(Cx<T> *v, Cx<T> *buf, int lane, co
     wave_lds_sync();
 }
 
-// Forward transform of registers in pass-1 layout; on return v[b R3 + r] is
-// point lane + 64 b + r M/R3.  Its plain pass-3 twiddles are looked up (one
-// forward transform per block).
-template <typename T, int M, typename W>
-__device__ __forceinline__ void wave_forward(Cx<T> *v, Cx<T> *buf, int lane, const W &w, const Twiddle<T> &tw)
+// One radix-4 pass of a 256-point forward transform held as 4 points per
+// lane, and the exchange to the next pass's inputs: outputs to points
+// (lane - k) 4 + k + r NS, k = lane mod NS; inputs lane + 64 r.
+template <typename T, int NS, typename F>
+__device__ __forceinline__ void fft256_pass(Cx<T> *y, Cx<T> *buf, int lane, F &&twiddle)
 {
-    using P = WavePlan<M>;
-    wave_passes12<T, M, false>(v, buf, lane, w);
+    const int k = lane & (NS - 1);
+    if constexpr (NS > 1) {
 #pragma unroll
-    for (int b = 0; b < W::B3; ++b) {
-#pragma unroll
-        for (int r = 1; r < P::R3; ++r) {
-            v[b * P::R3 + r] = cmul(v[b * P::R3 + r], tw(4 * r * (lane + 64 * b)));
-        }
-        mfcl::dftR<P::R3, false>(&v[b * P::R3]);
+        for (int r = 1; r < 4; ++r) { y[r] = cmul(y[r], twiddle(NS, r * k)); }
     }
+    mfcl::dftR<4, false>(y);
+    if constexpr (NS < 64) {
+        Cx<T> *p = buf + xpad((lane - k) * 4 + k);
+        const int low = ((lane - k) * 4 + k) & 15;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) { p[r * NS + ((low + r * NS) >> 4)] = y[r]; }
+        wave_lds_sync();
+        const Cx<T> *q = buf + xpad(lane);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) { y[r] = q[cpad(64 * r)]; }
+        wave_lds_sync();
+    }
+}
+
+// The points X_{G k + g}, k < 256, of the forward transform of the block
+// u_j = (d_j - i d_{j+M}) W_{4M}^j, M = 256 G, by one wave (residue g):
+//     y_j = W_{4M}^{j (4g+1)} sum_r (d_{j+256r} - i d_{j+M+256r}) c^r,
+//     c = W_{4M}^{256 (4g+1)} (its powers are table entries),  j < 256,
+// then a 256-point transform of y (lane: points lane + 64 q).  The residues
+// are independent, so the block's waves share one forward transform without
+// a barrier inside it (it is four times shorter than on one wave while the
+// others wait).  buf: 272 values of the wave's own; out[G k + g] = X.
+template <typename T, int G, typename F>
+__device__ __forceinline__ void forward_residue(F &&sample, int g, Cx<T> *buf, Cx<T> *out, int lane,
+                                                const Twiddle<T> &tw)
+{
+    constexpr int M = 256 * G;
+    Cx<T> y[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int j = lane + 64 * q;
+        Cx<T> s[G];
+#pragma unroll
+        for (int r = 0; r < G; ++r) { s[r] = {sample(j + 256 * r), -sample(j + M + 256 * r)}; }
+        // the sum by halves: r and r + h with c^h, h = G/2, ..., 2, 1
+#pragma unroll
+        for (int h = G / 2; h >= 1; h /= 2) {
+            const Cx<T> ch = tw.hi[(4 * h * (4 * g + 1)) & (16 * G - 1)];
+#pragma unroll
+            for (int r = 0; r < h; ++r) { s[r] = cadd(s[r], cmul(s[r + h], ch)); }
+        }
+        y[q] = cmul(s[0], tw(j * (4 * g + 1)));
+    }
+    // W_{4 NS}^e = W_{4M}^(e M / NS)
+    const auto twiddle = [&](int NS, int e) { return tw(e * (M / NS)); };
+    fft256_pass<T, 1>(y, buf, lane, twiddle);
+    fft256_pass<T, 4>(y, buf, lane, twiddle);
+    fft256_pass<T, 16>(y, buf, lane, twiddle);
+    fft256_pass<T, 64>(y, buf, lane, twiddle);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) { out[G * (lane + 64 * r) + g] = y[r]; }
 }
 
 // ---- half-size exchanges ------------------------------------------------
@@ -551,13 +657,13 @@ __device__ __forceinline__ void wave_exchange_half(Cx<T> *v, Cx<T> *buf, int lan
 }
 
 // wave_passes12 through a half buffer.
-template <typename T, int M, bool INV, typename W>
+template <typename T, int M, typename W>
 __device__ __forceinline__ void wave_passes12_half(Cx<T> *v, Cx<T> *buf, int lane, const W &tw)
 {
     using P = WavePlan<M>;
-    wave_butterflies<T, M, P::R1, INV, false>(v, nullptr);
+    wave_pass1<T, M>(v);
     wave_exchange_half<T, M, P::R1, 1, P::R2>(v, buf, lane);
-    wave_butterflies<T, M, P::R2, INV, true>(v, tw.w2);
+    wave_pass2<T, M>(v, tw);
     wave_exchange_half<T, M, P::R2, P::R1, P::R3>(v, buf, lane);
 }
 

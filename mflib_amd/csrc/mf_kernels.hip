@@ -498,8 +498,8 @@ __global__ __launch_bounds__(NT) void corr_kernel(const Item *__restrict__ items
 
 // ---------------------------------------------------------------------------
 // corr2_kernel: same contract as corr_kernel, built from wave-level FFTs.
-// Wave 0 computes the forward FFT while waves 1-3 build the normalisation
-// scale; then every wave takes whole template rows (one complex product per
+// The waves share the block's forward transform (a residue of bins each) and
+// the normalisation scale; then every wave takes whole template rows (one complex product per
 // bin in pass-1 registers, three register passes, epilogue straight from
 // pass-3 registers), so the row loop has no block barrier and a row's only
 // LDS traffic is the two exchanges between passes and the scale reads.  Rows are processed in groups of equal template length; the
@@ -595,21 +595,38 @@ __device__ __forceinline__ void fixup_row_wave(const T *raw, const T *sc, gptr<c
 // Shape of corr2_kernel<T, M>:
 //  - SHARED: a block-wide scale buffer for groups of rows of one template
 //    length (FP32 up to M = 1024, FP64 up to M = 512);
-//  - HALF (the larger blocks): every row computes its own scale, the
-//    per-wave exchange buffers are half size, the template spectrum of the
-//    next row is not prefetched into registers and the pass-3 twiddles come
-//    from the table.  That fits two blocks per CU in LDS and registers
-//    where the full layout fitted one;
+//  - HALF: half-size exchange buffers per wave (and a solo row's scale is
+//    computed half a block at a time);
+//  - W2LDS, W3REG: where the pass-2 and pass-3 twiddles live (WaveTwiddles);
 //  - TILE: samples per FP64 prefix-sum tile (FP32: 4, or 8 at M = 2048; FP64:
 //    16, whose windows sum whole tiles);
 //  - BLOCKS per CU that LDS and registers allow; the register budget is
 //    capped to match.
+// The kernel is bound by latency more than by any unit (53 % of the vector
+// issue slots and 29 % of LDS at two blocks per CU), so the shapes trade
+// registers and LDS for resident waves, and a row's spectrum is loaded when
+// its turn comes instead of a row ahead (32 registers at M = 1024): the
+// other waves cover the load.  Measured, correlation launch, of a shape at
+// two (M = 512 FP32: three) blocks with the spectrum a row ahead and full
+// exchange buffers -> this one:
+//   FP32 M = 1024, 24 channels x 16 rows x 8.64 M samples  6.90 -> 5.71 ms
+//        (two blocks without the prefetch 6.03, the pass-2 rows in registers
+//        at three blocks 6.04);
+//   FP32 M = 512, 4 channels x 256 rows x 2 M samples  5.94 -> 5.33 ms (half
+//        exchange buffers for five or six blocks spill: 6.5-6.9);
+//   FP64 M = 512, 24 channels x 1 row x 0.9 M samples  1.41 -> 1.02 ms (the
+//        pass-2 rows in registers 1.13).
+// M = 2048 stays at two blocks: its samples and spectrum alone take 32 KB
+// of LDS per block.
 template <typename T, int M>
 struct Corr2Shape {
+    static constexpr bool F64 = sizeof(T) == 8;
     static constexpr bool SHARED = corr2_shared_scale(static_cast<int>(sizeof(T)), M);
-    static constexpr bool HALF = !SHARED;
-    static constexpr int TILE = sizeof(T) == 4 ? (M >= 2048 ? 8 : 4) : 16;
-    static constexpr int BLOCKS = sizeof(T) * M <= 2048 ? 3 : 2;
+    static constexpr bool HALF = F64 || M >= 1024;
+    static constexpr bool W2LDS = F64 || M == 1024;
+    static constexpr bool W3REG = !F64 && M == 2048;
+    static constexpr int TILE = F64 ? 16 : (M >= 2048 ? 8 : 4);
+    static constexpr int BLOCKS = F64 ? (M == 512 ? 3 : 2) : (M == 512 ? 4 : M == 1024 ? 3 : 2);
 };
 
 template <typename T, int M, bool QUEUE>
@@ -637,20 +654,19 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
     __shared__ T raw[N];
     __shared__ Cx<T> Xs[M];
     __shared__ __align__(16) T sc[SHARED ? N : 1];
-    // one exchange buffer per wave (half size with HALF; then the first two
-    // together are the full buffer of the forward transform)
+    // one exchange buffer per wave (half size with HALF)
     __shared__ Cx<T> xb[NWAVE * XW];
-    // FP64 tile prefix sums; FP64 correlation also keeps the tile sums (FP32
-    // builds the prefix in place over the sums)
-    __shared__ double tp1[NTILE + 1];
-    __shared__ double tp2[NTILE + 1];
-    __shared__ double tsd1[sizeof(T) == 8 ? NTILE : 1];
-    __shared__ double tsd2[sizeof(T) == 8 ? NTILE : 1];
+    using W = WaveTwiddles<T, M, Shape::W2LDS, Shape::W3REG>;
+    __shared__ Cx<T> w2tab[W::TABLE];
+    // FP64 sums over tiles of TILE samples: FP32 correlation keeps their
+    // prefix sums, FP64 correlation the tile sums themselves
+    __shared__ __align__(16) double tp1[NTILE + 1];
+    __shared__ __align__(16) double tp2[NTILE + 1];
     __shared__ Cx<T> twlo[64];
     __shared__ Cx<T> twhi[N / 32];
     __shared__ double red[NWAVE];
-    double *ts1 = sizeof(T) == 8 ? tsd1 : tp1;
-    double *ts2 = sizeof(T) == 8 ? tsd2 : tp2;
+    __shared__ double tot1[NWAVE], tot2[NWAVE];
+    const double *ts1 = tp1, *ts2 = tp2;
 
     const Item item = items[blockIdx.x];
     if (item.nRows == 0) { return; }  // an empty item that keeps the XCD order
@@ -676,77 +692,116 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
     for (int i = tid; i < N / 32; i += NT) { twhi[i] = twhiG[i]; }
     const Twiddle<T> tw{twlo, twhi};
 
-    // A. load, anchor, tile sums, energy
-    const gptr<const T> x = to_global(static_cast<const T *>(sg.x));
+    // A. load, anchor, tile sums, energy.  Each thread takes SPT consecutive
+    // samples, so tile sums and their scan stay in registers and DPP moves.
+    // The anchor a removes the block's offset: any value near the samples
+    // will do (the templates have zero mean, and the error model takes the
+    // energy about a), so every wave takes the same mean of 64 samples
+    // spread over the block, and no barrier is needed before the sums.
+    const gptr<const T> x = to_global(static_cast<const T *>(sg.x)) + base;
     const int nSamp = static_cast<int>(min(static_cast<long long>(N), sg.n - base));
+    const T spread = x[min(lane * (N / 64), nSamp - 1)];
     T v0[SPT];
-    double s = 0;
+    const int j0 = tid * SPT;
+    if (nSamp == N) {
+        constexpr int VL = 16 / static_cast<int>(sizeof(T));
+        typedef T VecU __attribute__((ext_vector_type(VL), aligned(sizeof(T))));  // base is not 16-byte aligned
 #pragma unroll
-    for (int q = 0; q < SPT; ++q) {
-        const int j = tid + q * NT;
-        const T val = (j < nSamp) ? x[base + j] : T(0);
-        v0[q] = val;
-        raw[j] = val;
-        s += static_cast<double>(val);
-    }
-    const double a = uniform(block_sum<NT>(s, red) / nSamp);  // scalar registers: used by every row
-    const T aT = static_cast<T>(a);
-    double e = 0;
+        for (int q = 0; q < SPT; q += VL) {
+            const VecU t = *reinterpret_cast<const __attribute__((address_space(1))) VecU *>(x + j0 + q);
 #pragma unroll
-    for (int q = 0; q < SPT; ++q) {
-        const int j = tid + q * NT;
-        const bool valid = j < nSamp;
-        const double d = valid ? static_cast<double>(v0[q]) - a : 0.0;
-        double t1 = d, t2 = d * d;
-        e += t2;
-#pragma unroll
-        for (int o = TILE / 2; o > 0; o >>= 1) {
-            t1 += __shfl_xor(t1, o, 64);
-            t2 += __shfl_xor(t2, o, 64);
+            for (int e = 0; e < VL; ++e) { v0[q + e] = t[e]; }
         }
-        if ((tid & (TILE - 1)) == 0) {
-            ts1[j / TILE] = t1;
-            ts2[j / TILE] = t2;
+    } else {
+#pragma unroll
+        for (int q = 0; q < SPT; ++q) { v0[q] = j0 + q < nSamp ? x[j0 + q] : T(0); }
+    }
+    const T aT = read_lane(wave_scan_sum(spread * T(1.0 / 64)), 63);
+    const double a = static_cast<double>(aT);
+    double l1[SPT / TILE + 1], l2[SPT / TILE + 1];  // running sums at the thread's tile starts, then its totals
+    {
+        double r1 = 0, r2 = 0;
+#pragma unroll
+        for (int q = 0; q < SPT; ++q) {
+            if (q % TILE == 0) {
+                l1[q / TILE] = r1;
+                l2[q / TILE] = r2;
+            }
+            const double d = j0 + q < nSamp ? static_cast<double>(v0[q]) - a : 0.0;
+            r1 += d;
+            r2 += d * d;
+            raw[j0 + q] = v0[q];
+        }
+        l1[SPT / TILE] = r1;
+        l2[SPT / TILE] = r2;
+    }
+    const double t1 = l1[SPT / TILE], t2 = l2[SPT / TILE];  // the thread's totals
+    const double i1 = wave_scan_sum(t1), i2 = wave_scan_sum(t2);
+    if (lane == 63) {
+        tot1[wave] = i1;
+        tot2[wave] = i2;
+    }
+    if constexpr (sizeof(T) == 8) {
+        // a tile is TILE / SPT neighbouring threads
+        double u1 = t1, u2 = t2;
+#pragma unroll
+        for (int o = TILE / SPT / 2; o > 0; o >>= 1) {
+            u1 += __shfl_xor(u1, o, 64);
+            u2 += __shfl_xor(u2, o, 64);
+        }
+        if (tid % (TILE / SPT) == 0) {
+            tp1[j0 / TILE] = u1;
+            tp2[j0 / TILE] = u2;
         }
     }
-    const double energy = block_sum<NT>(e, red);
-    tile_prefix<NTILE>(ts1, ts2, tp1, tp2, tid);  // in place for FP32 (each lane reads its tiles first)
-    __syncthreads();
-    const double rmsBlk = sqrt(energy / nSamp);
+    __syncthreads();  // samples, wave totals and twiddle tables are in LDS
+    W::fill(w2tab, tid, NT, tw);
+    double energy = 0;
+    {
+        double o1 = 0, o2 = 0;
+#pragma unroll
+        for (int w = 0; w < NWAVE; ++w) {
+            if (w == wave) {
+                o1 += i1 - t1;
+                o2 = energy + (i2 - t2);
+            } else if (w < wave) {
+                o1 += tot1[w];
+            }
+            energy += tot2[w];
+        }
+        if constexpr (sizeof(T) == 4) {
+#pragma unroll
+            for (int q = 0; q < SPT / TILE; ++q) {
+                tp1[j0 / TILE + q] = o1 + l1[q];
+                tp2[j0 / TILE + q] = o2 + l2[q];
+            }
+            if (tid == NT - 1) {
+                tp1[NTILE] = o1 + t1;
+                tp2[NTILE] = o2 + t2;
+            }
+        }
+    }
+    // a block with a NaN or infinite sample has no usable transform: every
+    // window is recomputed exactly
+    const double rmsBlk = energy < INFINITY ? sqrt(energy / nSamp) : INFINITY;
     const double noise = uniform(kNoiseK / Eps<T>::rhoTol * Eps<T>::value * sqrt(static_cast<double>(LOGN)) *
                                  static_cast<double>(sg.hmax) * rmsBlk);
-    WaveTwiddles<T, M, !HALF> wt;
-    wt.initPass2(lane, tw);
+    // B. forward transform of u_j = (d_j - i d_{j+M}) W_{4M}^j into Xs, its
+    // residues of bins shared out over the waves
+    {
+        constexpr int G = M / 256;
+        const auto sample = [&](int j) { return j < nSamp ? static_cast<T>(raw[j] - aT) : T(0); };
+        for (int g = wave; g < G; g += NWAVE) { forward_residue<T, G>(sample, g, xb + wave * XW, Xs, lane, tw); }
+    }
+    __syncthreads();  // Xs and the tile sums are complete
+    W wt;
+    wt.init(lane, tw, w2tab);
     Cx<T> v[Q];
 
-    // B. forward transform of u_j = (x_j - i x_{j+M}) W_{4M}^j into Xs (wave
-    // 0, full buffer); the lane's points are lane + 64 q
-    auto forwardFft = [&]() {
-        const auto sample = [&](int j) { return j < nSamp ? static_cast<T>(raw[j] - aT) : T(0); };
-#pragma unroll
-        for (int q = 0; q < Q; ++q) {
-            const int j = lane + 64 * q;
-            // pass-1 register of point j = lane + 64 b + r M/R1
-            const int reg = (q % (Q / P::R1)) * P::R1 + q / (Q / P::R1);
-            v[reg] = cmul(Cx<T>{sample(j), -sample(j + M)}, tw(j));
-        }
-        wave_forward<T, M>(v, xb, lane, wt, tw);
-#pragma unroll
-        for (int b = 0; b < Q / P::R3; ++b) {
-#pragma unroll
-            for (int r = 0; r < P::R3; ++r) { Xs[lane + 64 * b + r * (M / P::R3)] = v[b * P::R3 + r]; }
-        }
-    };
-
     // C. one template row on this wave, in two halves.  startRow: spectral
-    // product and the three register passes (the result stays in v).  finishRow: the row's scale when it has no shared one,
-    // then the normalisation epilogue straight from the pass-3 registers.
-    // A wave's row sequence runs start(r0), then for each next row r:
-    // finish(previous), start(r), and finally finish(last).  start(r)
-    // loads the spectrum of the row after r once its product is done, so
-    // the load is in flight through r's transform and epilogue; the
-    // epilogue issues the same (range-checked) stores on every path, so
-    // the wait for that spectrum never waits for those stores.
+    // product and the three register passes (the result stays in v).
+    // finishRow: the row's scale when it has no shared one, then the
+    // normalisation epilogue straight from the pass-3 registers.
     Cx<T> hk[Q];  // template spectrum at the lane's points lane + 64 q
     auto loadH = [&](const void *Hp) {
         const gptr<const Cx<T>> H = to_global(static_cast<const Cx<T> *>(Hp));
@@ -756,26 +811,19 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
     auto rowValid = [&](const Row &row) {
         return static_cast<int>(max(0ll, min(static_cast<long long>(sg.L), row.nOut - base)));
     };
-    constexpr bool PREFETCH = !HALF;
-    auto startRow = [&](const Row &row, const void *nextH) {
-        if (rowValid(row) == 0) {
-            if (PREFETCH) { loadH(nextH); }
-            return;
-        }
-        if (!PREFETCH) { loadH(row.H); }
+    auto startRow = [&](const Row &row) {
+        if (rowValid(row) == 0) { return; }
+        loadH(row.H);
         Cx<T> *buf = xb + wave * XW;
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
             const int reg = (q % (Q / P::R1)) * P::R1 + q / (Q / P::R1);
             v[reg] = cmul(Xs[lane + 64 * q], hk[q]);
         }
-        // the next row's spectrum is in flight through this row's transform
-        // and epilogue
-        if (PREFETCH) { loadH(nextH); }
         if constexpr (HALF) {
-            wave_passes12_half<T, M, true>(v, buf, lane, wt);
+            wave_passes12_half<T, M>(v, buf, lane, wt);
         } else {
-            wave_passes12<T, M, true>(v, buf, lane, wt);
+            wave_passes12<T, M>(v, buf, lane, wt);
         }
         wave_pass3_inverse<T, M>(v, wt);
     };
@@ -930,39 +978,17 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
         while (g1 < rowEnd && rows[g1].Lt == rows[g0].Lt) { ++g1; }
         return g1;
     };
-    // wave 0 transforms while waves 1..3 build the first group's scale, if
-    // it is a shared one
-    const bool firstShared = SHARED && groupEnd(sg.rowBegin) - sg.rowBegin >= kCorr2SharedGroup;
-    int myFlags = 0;
-    if (wave == 0) {
-        forwardFft();
-    } else if (firstShared) {
-        myFlags = compute_scale<T, TILE, 1, QUEUE>(raw, ts1, ts2, tp1, tp2, sc, a, nValidSeg, rows[sg.rowBegin].Lt,
-                                                   noise, tid - 64, NT - 64);
-    }
-    // pass-3 twiddles only now: the forward transform is over, and so is its
-    // need of registers
-    wt.initPass3(lane, tw);
-    if (!firstShared) { __syncthreads(); }
     if constexpr (SHARED) {
         for (int g0 = sg.rowBegin; g0 < rowEnd;) {
             const int g1 = groupEnd(g0);
             if (g1 - g0 >= kCorr2SharedGroup) {
-                if (g0 != sg.rowBegin) {
-                    myFlags = compute_scale<T, TILE, 1, QUEUE>(raw, ts1, ts2, tp1, tp2, sc, a, nValidSeg, rows[g0].Lt,
-                                                               noise, tid, NT);
-                }
-                const double flagSum = uniform(block_sum<NT>(static_cast<double>(myFlags), red));  // scalar registers
-                const bool anyFlag = flagSum > 0.0;
-                int r = g0 + wave;
-                if (r < g1) {
-                    if (PREFETCH) { loadH(rows[r].H); }
-                    startRow(rows[r], rows[r + NWAVE < g1 ? r + NWAVE : r].H);
-                    for (int rn = r + NWAVE; rn < g1; rn += NWAVE) {
-                        finishRow(rows[r], r, sc, anyFlag, flagSum);
-                        startRow(rows[rn], rows[rn + NWAVE < g1 ? rn + NWAVE : rn].H);
-                        r = rn;
-                    }
+                const int myFlags = compute_scale<T, TILE, 1, QUEUE>(raw, ts1, ts2, tp1, tp2, sc, a, nValidSeg,
+                                                                     rows[g0].Lt, noise, tid, NT);
+                const bool anyFlag = __syncthreads_or(myFlags) != 0;
+                double flagSum = 0;
+                if (QUEUE && anyFlag) { flagSum = uniform(block_sum<NT>(static_cast<double>(myFlags), red)); }
+                for (int r = g0 + wave; r < g1; r += NWAVE) {
+                    startRow(rows[r]);
                     finishRow(rows[r], r, sc, anyFlag, flagSum);
                 }
                 __syncthreads();  // sc is rebuilt for the next group
@@ -989,18 +1015,8 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
             if (((sk++) & (NWAVE - 1)) == wave) { return r; }
         }
     };
-    int cur = nextSolo();
-    if (cur >= 0) {
-        if (PREFETCH) { loadH(rows[cur].H); }
-        int nx = nextSolo();
-        startRow(rows[cur], rows[nx >= 0 ? nx : cur].H);
-        while (nx >= 0) {
-            const int nn = nextSolo();
-            finishRow(rows[cur], cur, nullptr, false, 0.0);
-            startRow(rows[nx], rows[nn >= 0 ? nn : nx].H);
-            cur = nx;
-            nx = nn;
-        }
+    for (int cur = nextSolo(); cur >= 0; cur = nextSolo()) {
+        startRow(rows[cur]);
         finishRow(rows[cur], cur, nullptr, false, 0.0);
     }
 }

@@ -656,6 +656,49 @@ __device__ __forceinline__ void wave_exchange_half(Cx<T> *v, Cx<T> *buf, int lan
     for (int i = 0; i < Q; ++i) { v[i] = u[i]; }
 }
 
+// Exchange of one component at a time through a buffer of M values of T
+// (half the bytes of a complex buffer, all lanes busy, where half buffers
+// with one butterfly per lane leave half the lanes idle).  One spare slot
+// every 8 values: 8 consecutive values per lane then spread over the banks.
+template <int M>
+struct XSplit {
+    static constexpr int size = M + M / 8;  // values of T
+};
+template <typename T, int M, int RS, int NS, int RL>
+__device__ __forceinline__ void wave_exchange_split(Cx<T> *v, T *buf, int lane)
+{
+    static_assert(M == 64 * RS && RS == 8 && RL == 8 && (NS == 1 || NS % 8 == 0), "one radix-8 butterfly per lane");
+    const int k = lane & (NS - 1);
+    const int dst = (lane - k) * RS + k;
+    T *p = buf + dst + (dst >> 3);
+    const T *q = buf + lane + (lane >> 3);
+    // value r goes to dst + r NS: the pad grows by r NS / 8 (NS = 1: not
+    // within a lane's 8)
+    constexpr int step = NS + NS / 8;
+#pragma unroll
+    for (int r = 0; r < RS; ++r) { p[r * step] = v[r].x; }
+    wave_lds_sync();
+    T x[RL];
+#pragma unroll
+    for (int r = 0; r < RL; ++r) { x[r] = q[72 * r]; }
+    wave_lds_sync();
+#pragma unroll
+    for (int r = 0; r < RS; ++r) { p[r * step] = v[r].y; }
+    wave_lds_sync();
+#pragma unroll
+    for (int r = 0; r < RL; ++r) { v[r] = {x[r], q[72 * r]}; }
+    wave_lds_sync();
+}
+template <typename T, int M, typename W>
+__device__ __forceinline__ void wave_passes12_split(Cx<T> *v, T *buf, int lane, const W &tw)
+{
+    using P = WavePlan<M>;
+    wave_pass1<T, M>(v);
+    wave_exchange_split<T, M, P::R1, 1, P::R2>(v, buf, lane);
+    wave_pass2<T, M>(v, tw);
+    wave_exchange_split<T, M, P::R2, P::R1, P::R3>(v, buf, lane);
+}
+
 // wave_passes12 through a half buffer.
 template <typename T, int M, typename W>
 __device__ __forceinline__ void wave_passes12_half(Cx<T> *v, Cx<T> *buf, int lane, const W &tw)

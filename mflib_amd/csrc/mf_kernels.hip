@@ -297,8 +297,8 @@ __device__ __forceinline__ int wave_row_scale(const float *raw, const double *tp
 constexpr int kDenseFlags = 16;
 
 // Exact FP64 two-pass Pearson of the window at wi, by one lane.
-template <typename T>
-__device__ __forceinline__ double exact_window(const T *raw, int wi, gptr<const double> tmpl, int Lt)
+template <typename XPtr>
+__device__ __forceinline__ double exact_window(XPtr raw, int wi, gptr<const double> tmpl, int Lt)
 {
     double sm = 0;
     for (int mm = 0; mm < Lt; ++mm) { sm += static_cast<double>(raw[wi + mm]); }
@@ -463,7 +463,7 @@ __global__ __launch_bounds__(NT) void corr_kernel(const Item *__restrict__ items
                 nFlag += __popcll(m);
                 nCanc += __popcll(__ballot(fl && isinf(sc[i])));
                 if (__popcll(m) >= kDenseFlags) {
-                    if (fl) { out[i] = static_cast<T>(exact_window<T>(raw, i, to_global(row.tmpl), Lt)); }
+                    if (fl) { out[i] = static_cast<T>(exact_window(raw, i, to_global(row.tmpl), Lt)); }
                     continue;
                 }
                 while (m != 0ull) {
@@ -507,25 +507,24 @@ __global__ __launch_bounds__(NT) void corr_kernel(const Item *__restrict__ items
 // ---------------------------------------------------------------------------
 
 // In-place exact recomputation of the flagged outputs of one chunk of 64
-// (mask m, output w0 + lane for this lane) of a row, sc[i] < 0 flagging
-// output i (see scale_exact): a noise flag (-f) keeps the window's scale f
+// (mask m, output w0 + lane for this lane) of a row, the lane's s < 0
+// flagging its output (see scale_exact): a noise flag (-f) keeps the window's scale f
 // and recomputes the numerator exactly in FP64 from the anchored samples,
 // sum_m t[m] (x[i+m] - a) (the template has zero mean, so the window mean
 // drops out of the numerator); -infinity recomputes the two-pass Pearson
 // value.  Many flags: one lane per window; few: the wave on each window.
-template <typename T>
-__device__ __forceinline__ void fixup_chunk(const T *raw, const T *sc, gptr<const double> tmpl, int Lt, gptr<T> out,
-                                            int w0, int nv, int lane, double a, unsigned long long m)
+template <typename T, typename XPtr>
+__device__ __forceinline__ void fixup_chunk(XPtr raw, T s, gptr<const double> tmpl, int Lt, gptr<T> out, int w0,
+                                            int lane, double a, unsigned long long m)
 {
     const int i = w0 + lane;
-    const T s = i < nv ? sc[i] : T(1);
     const bool fl = s < T(0);
     if (__popcll(m) >= kDenseFlags) {
         // many flagged windows (a gap, a loud stretch): one lane per window
         if (fl) {
             double rho;
             if (isinf(s)) {
-                rho = exact_window<T>(raw, i, tmpl, Lt);
+                rho = exact_window(raw, i, tmpl, Lt);
             } else {
                 double dn = 0;
                 for (int mm = 0; mm < Lt; ++mm) { dn = fma(tmpl[mm], static_cast<double>(raw[i + mm]) - a, dn); }
@@ -540,7 +539,7 @@ __device__ __forceinline__ void fixup_chunk(const T *raw, const T *sc, gptr<cons
         const int b = __ffsll(static_cast<long long>(m)) - 1;
         m &= m - 1ull;
         const int wi = w0 + b;
-        const T sw = sc[wi];
+        const T sw = read_lane(s, b);
         double rho;
         if (isinf(sw)) {
             double sm = 0;
@@ -570,8 +569,8 @@ __device__ __forceinline__ void fixup_chunk(const T *raw, const T *sc, gptr<cons
 // Flagged outputs [first, nv) of one row (one wave), sc[i - first] < 0
 // flagging output i (see scale_exact), recomputed in place chunk by chunk;
 // their count goes to the window statistics.
-template <typename T>
-__device__ __forceinline__ void fixup_row_wave(const T *raw, const T *sc, gptr<const double> tmpl, int Lt,
+template <typename T, typename XPtr>
+__device__ __forceinline__ void fixup_row_wave(XPtr raw, const T *sc, gptr<const double> tmpl, int Lt,
                                                gptr<T> out, int nv, int lane, double a, int first,
                                                unsigned long long *flagged)
 {
@@ -584,7 +583,7 @@ __device__ __forceinline__ void fixup_row_wave(const T *raw, const T *sc, gptr<c
         const unsigned long long m = __ballot(fl);
         nFlag += __popcll(m);
         nCanc += __popcll(__ballot(fl && isinf(s)));
-        if (m != 0ull) { fixup_chunk<T>(raw, sc, tmpl, Lt, out, w0, nv, lane, a, m); }
+        if (m != 0ull) { fixup_chunk<T>(raw, s, tmpl, Lt, out, w0, lane, a, m); }
     }
     if (flagged != nullptr && nFlag != 0u && lane == 0) {
         atomicAdd(flagged, static_cast<unsigned long long>(nFlag));
@@ -626,7 +625,13 @@ struct Corr2Shape {
     static constexpr bool W2LDS = F64 || M == 1024;
     static constexpr bool W3REG = !F64 && M == 2048;
     static constexpr int TILE = F64 ? 16 : (M >= 2048 ? 8 : 4);
+    static constexpr bool PREFIX = !F64 && M == 512;
     static constexpr int BLOCKS = F64 ? (M == 512 ? 3 : 2) : (M == 512 ? 4 : M == 1024 ? 3 : 2);
+};
+
+// FP64 prefix sums of d and d^2 at one sample.
+struct __align__(16) Prefix {
+    double s1, s2;
 };
 
 template <typename T, int M, bool QUEUE>
@@ -638,6 +643,7 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
 {
     using Shape = Corr2Shape<T, M>;
     constexpr int N = 2 * M;
+    constexpr bool PREFIX = Shape::PREFIX;
     constexpr int TILE = Shape::TILE;
     constexpr bool SHARED = Shape::SHARED;
     constexpr bool HALF = Shape::HALF;
@@ -647,11 +653,23 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
     constexpr int Q = M / 64;
     constexpr int NWAVE = NT / 64;
     constexpr int XH = XHalf<M>::size;
-    constexpr int XW = HALF ? XH : XBuf<M>::size;  // exchange buffer of one wave
+    // exchange buffer of one wave
+    constexpr int XW = PREFIX ? XSplit<M>::size / 2 : HALF ? XH : XBuf<M>::size;
     using P = WavePlan<M>;
-    static_assert(N % NT == 0 && NWAVE == 4, "block shape");
+    static_assert(N % NT == 0, "block shape");
     static_assert(2 * XH == XBuf<M>::size, "two half buffers make one full buffer");
-    __shared__ T raw[N];
+    // PREFIX: the FP64 prefix sums at every sample, one spare entry per 16 so
+    // that the 4 consecutive entries a thread writes spread over the LDS
+    // banks, and GROUP - 1 entries past the end, which the reads for outputs
+    // past a row's last may touch.  The block's samples lie there first (the
+    // forward transform reads them).
+    constexpr int GROUP = 128;
+    constexpr auto ppad = [](int i) { return i + (i >> 4); };
+    constexpr int NP = PREFIX ? N + GROUP + (N + GROUP) / 16 : 1;
+    __shared__ Prefix pf[NP];
+    __shared__ unsigned eqw[PREFIX ? N / 32 : 1];  // bit j: sample j equals sample j + 1
+    __shared__ T rawBuf[PREFIX ? 1 : N];
+    T *raw = PREFIX ? reinterpret_cast<T *>(pf) : rawBuf;
     __shared__ Cx<T> Xs[M];
     __shared__ __align__(16) T sc[SHARED ? N : 1];
     // one exchange buffer per wave (half size with HALF)
@@ -660,8 +678,8 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
     __shared__ Cx<T> w2tab[W::TABLE];
     // FP64 sums over tiles of TILE samples: FP32 correlation keeps their
     // prefix sums, FP64 correlation the tile sums themselves
-    __shared__ __align__(16) double tp1[NTILE + 1];
-    __shared__ __align__(16) double tp2[NTILE + 1];
+    __shared__ __align__(16) double tp1[PREFIX ? 1 : NTILE + 1];
+    __shared__ __align__(16) double tp2[PREFIX ? 1 : NTILE + 1];
     __shared__ Cx<T> twlo[64];
     __shared__ Cx<T> twhi[N / 32];
     __shared__ double red[NWAVE];
@@ -718,24 +736,25 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
     }
     const T aT = read_lane(wave_scan_sum(spread * T(1.0 / 64)), 63);
     const double a = static_cast<double>(aT);
-    double l1[SPT / TILE + 1], l2[SPT / TILE + 1];  // running sums at the thread's tile starts, then its totals
+    constexpr int STEP = PREFIX ? 1 : TILE;         // samples between the sums kept
+    double l1[SPT / STEP + 1], l2[SPT / STEP + 1];  // running sums there, then the thread's totals
     {
         double r1 = 0, r2 = 0;
 #pragma unroll
         for (int q = 0; q < SPT; ++q) {
-            if (q % TILE == 0) {
-                l1[q / TILE] = r1;
-                l2[q / TILE] = r2;
+            if (q % STEP == 0) {
+                l1[q / STEP] = r1;
+                l2[q / STEP] = r2;
             }
             const double d = j0 + q < nSamp ? static_cast<double>(v0[q]) - a : 0.0;
             r1 += d;
             r2 += d * d;
             raw[j0 + q] = v0[q];
         }
-        l1[SPT / TILE] = r1;
-        l2[SPT / TILE] = r2;
+        l1[SPT / STEP] = r1;
+        l2[SPT / STEP] = r2;
     }
-    const double t1 = l1[SPT / TILE], t2 = l2[SPT / TILE];  // the thread's totals
+    const double t1 = l1[SPT / STEP], t2 = l2[SPT / STEP];  // the thread's totals
     const double i1 = wave_scan_sum(t1), i2 = wave_scan_sum(t2);
     if (lane == 63) {
         tot1[wave] = i1;
@@ -757,8 +776,8 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
     __syncthreads();  // samples, wave totals and twiddle tables are in LDS
     W::fill(w2tab, tid, NT, tw);
     double energy = 0;
+    double o1 = 0, o2 = 0;  // the sums before the thread's first sample
     {
-        double o1 = 0, o2 = 0;
 #pragma unroll
         for (int w = 0; w < NWAVE; ++w) {
             if (w == wave) {
@@ -769,7 +788,7 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
             }
             energy += tot2[w];
         }
-        if constexpr (sizeof(T) == 4) {
+        if constexpr (sizeof(T) == 4 && !PREFIX) {
 #pragma unroll
             for (int q = 0; q < SPT / TILE; ++q) {
                 tp1[j0 / TILE + q] = o1 + l1[q];
@@ -793,7 +812,30 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
         const auto sample = [&](int j) { return j < nSamp ? static_cast<T>(raw[j] - aT) : T(0); };
         for (int g = wave; g < G; g += NWAVE) { forward_residue<T, G>(sample, g, xb + wave * XW, Xs, lane, tw); }
     }
-    __syncthreads();  // Xs and the tile sums are complete
+    __syncthreads();  // Xs and the tile sums are complete; with PREFIX, the samples are read
+    if constexpr (PREFIX) {
+#pragma unroll
+        for (int q = 0; q < SPT; ++q) { pf[ppad(j0 + q)] = Prefix{o1 + l1[q], o2 + l2[q]}; }
+        // past the samples: the total, which the thread of the last sample has
+        if (wave == NWAVE - 1) {
+            const Prefix total{read_lane(o1 + t1, 63), read_lane(o2 + t2, 63)};
+            for (int i = N + lane; i < N + GROUP; i += 64) { pf[ppad(i)] = total; }
+        }
+        // equal-neighbour bits, SPT per thread (the last sample has no
+        // neighbour), two threads to a byte
+        static_assert(!PREFIX || SPT == 4, "half a byte of bits per thread");
+        const T next = __shfl_down(v0[0], 1, 64);
+        unsigned bits = 0;
+#pragma unroll
+        for (int q = 0; q < SPT; ++q) {
+            const bool eq = v0[q] == (q + 1 < SPT ? v0[q + 1] : next);
+            bits |= (eq && (q + 1 < SPT || lane < 63) ? 1u : 0u) << q;
+        }
+        if (lane == 63 && j0 + SPT < nSamp && v0[SPT - 1] == x[j0 + SPT]) { bits |= 1u << (SPT - 1); }
+        bits |= __shfl_down(bits, 1, 64) << SPT;
+        if ((tid & 1) == 0) { reinterpret_cast<unsigned char *>(eqw)[tid / 2] = static_cast<unsigned char>(bits); }
+        __syncthreads();
+    }
     W wt;
     wt.init(lane, tw, w2tab);
     Cx<T> v[Q];
@@ -820,7 +862,9 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
             const int reg = (q % (Q / P::R1)) * P::R1 + q / (Q / P::R1);
             v[reg] = cmul(Xs[lane + 64 * q], hk[q]);
         }
-        if constexpr (HALF) {
+        if constexpr (PREFIX) {
+            wave_passes12_split<T, M>(v, reinterpret_cast<T *>(buf), lane, wt);
+        } else if constexpr (HALF) {
             wave_passes12_half<T, M>(v, buf, lane, wt);
         } else {
             wave_passes12<T, M>(v, buf, lane, wt);
@@ -856,6 +900,94 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
             }
         }
     };
+    // PREFIX: the scale of output i of a row, and its flag.  With S1, S2 the
+    // window's sums of d = x - a and d^2 (differences of the prefix sums) and
+    // den2 = Lt S2 - S1^2, a window is flagged when den2 is not above thr: the
+    // larger of the FFT noise bound and kc = 2e-9 Lt^2 E (E the block's sum of
+    // d^2, which bounds S2): below that the prefix sums' rounding, about
+    // 1e-15 Lt E, and the subtraction could cost digits.
+    struct RowScale {
+        double lt, kc;
+        float thr, sqrtLt;
+    };
+    const double energyU = uniform(energy);
+    const auto rowScale = [&](int Lt) {
+        RowScale rs;
+        rs.lt = static_cast<double>(Lt);
+        const double root = sqrt(rs.lt);
+        rs.kc = 2.0e-9 * rs.lt * rs.lt * energyU;
+        rs.thr = static_cast<float>(fmax(rs.kc, rs.lt * noise * noise));
+        rs.sqrtLt = static_cast<float>(root);
+        return rs;
+    };
+    const auto windowDen2 = [](Prefix lo, Prefix hi, double lt) {
+        const double s1 = hi.s1 - lo.s1, s2 = hi.s2 - lo.s2;
+        return fma(-s1, s1, lt * s2);
+    };
+    const auto scaleOf = [](float d2, float sqrtLt) {  // sqrt(Lt / den2): rsqrt and one Newton step
+        const float y = __builtin_amdgcn_rsqf(d2);
+        return (sqrtLt * y) * fmaf(-0.5f * d2, y * y, 1.5f);
+    };
+    // The normalisation epilogue of a solo row straight from the prefix table
+    // (two 16-byte LDS reads and about 14 vector instructions per output, no
+    // chains, no scale buffer, and none of it for outputs past the row's end);
+    // true if a window was flagged (written as NaN).
+    const auto prefixEpilogue = [&](int Lt, T *outRow, int nvRow) {
+        const __amdgpu_buffer_rsrc_t rs = buffer_rsrc(outRow, static_cast<int>(sizeof(T)) * nvRow);
+        const RowScale sc1 = rowScale(Lt);
+        const Prefix *lo = pf + ppad(lane);
+        const Prefix *hi = pf + ppad(lane + Lt);  // + ppad(k) for outputs lane + k, k a multiple of 64
+        unsigned long long any = 0;
+        constexpr int GB = GROUP / 64;
+        // the groups of GROUP outputs that hold valid ones
+#pragma unroll
+        for (int g = 0; g < N / GROUP; ++g) {
+            if (g * GROUP < nvRow) {
+                unsigned long long flags = 0;
+#pragma unroll
+                for (int k = 0; k < GB; ++k) {
+                    const int t = (g * GB + k) % Q;  // the lane's point lane + 64 t
+                    const bool upper = g * GB + k >= Q;
+                    const int reg = (t % B3) * P::R3 + t / B3;
+                    const int off = 64 * (g * GB + k);
+                    const float d2 = static_cast<float>(windowDen2(lo[ppad(off)], hi[ppad(off)], sc1.lt));
+                    const bool flag = !(d2 > sc1.thr);
+                    const float f = flag ? __builtin_nanf("") : scaleOf(d2, sc1.sqrtLt);
+                    flags |= __ballot(flag && lane + off < nvRow);
+                    buffer_store(static_cast<T>((upper ? -v[reg].y : v[reg].x) * f), rs,
+                                 static_cast<int>(sizeof(T)) * (lane + off));
+                }
+                any |= flags;
+            }
+        }
+        return any != 0;
+    };
+    // PREFIX: the scales of the block's outputs for a group of rows of one
+    // length, as compute_scale, but (QUEUE) with 0 for an exactly constant
+    // window (whose value is 0, if the transform is finite).  Returns this thread's
+    // packed flag counts, and kFix for a flagged window left to recompute.
+    constexpr int kFix = 1 << 30;
+    const auto prefixScale = [&](int Lt) {
+        const RowScale rs = rowScale(Lt);
+        int flags = 0;
+        for (int i = tid; i < nValidSeg; i += NT) {
+            const double den2 = windowDen2(pf[ppad(i)], pf[ppad(i + Lt)], rs.lt);
+            const float d2 = static_cast<float>(den2);
+            T f = static_cast<T>(scaleOf(d2, rs.sqrtLt));
+            if (!(d2 > rs.thr)) {
+                const bool canc = !(den2 > rs.kc);
+                flags += canc ? (1 << 16) + 1 : 1;
+                if (QUEUE && canc && energyU < INFINITY && constant_window(eqw, i, Lt)) {
+                    f = T(0);
+                } else {
+                    flags |= kFix;
+                    f = QUEUE ? static_cast<T>(__builtin_nanf("")) : canc ? scale_exact<T>() : -f;
+                }
+            }
+            sc[i] = f;
+        }
+        return flags;
+    };
     using Half0 = std::integral_constant<int, 0>;
     using Half1 = std::integral_constant<int, 1>;
     // sharedScale is the row's block-shared scale, or null: the wave then
@@ -881,24 +1013,57 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
             if (nc != 0ull) { atomicAdd(sg.flagged + 1, nc); }
         }
     };
-    auto finishRow = [&](const Row &row, int rowIdx, const T *sharedScale, bool anyFlagShared, double flagSum) {
+    auto finishRow = [&](const Row &row, int rowIdx, const T *sharedScale, int anyShared, double flagSum) {
         const int nvRow = rowValid(row);
         T *outRow = static_cast<T *>(row.out) + base;
         if (sharedScale != nullptr) {
             epilogueHalf(Half0{}, sharedScale, 0, outRow, nvRow);
             epilogueHalf(Half1{}, sharedScale, 0, outRow, nvRow);
-            if (anyFlagShared && nvRow > 0) {
+            if (anyShared != 0 && nvRow > 0) {
                 if constexpr (QUEUE) {
-                    recordRow(rowIdx, 0, nvRow);
+                    if ((anyShared & kFix) != 0) { recordRow(rowIdx, 0, nvRow); }
                     if (lane == 0) {
                         const unsigned long long packed = static_cast<unsigned long long>(flagSum);
                         countFlags(packed & 0xffffull, packed >> 16);
                     }
                 } else {
-                    fixup_row_wave<T>(raw, sharedScale, to_global(row.tmpl), row.Lt, to_global(outRow), nvRow, lane,
-                                      a, 0, sg.flagged);
+                    fixup_row_wave<T>(x, sharedScale, to_global(row.tmpl), row.Lt, to_global(outRow), nvRow, lane, a, 0,
+                                      sg.flagged);
                 }
             }
+            return;
+        }
+        if constexpr (PREFIX) {
+            if (nvRow == 0 || !prefixEpilogue(row.Lt, outRow, nvRow)) { return; }
+            // flagged windows: counted; exactly constant ones are 0 at once;
+            // the others are recorded (QUEUE) or recomputed here
+            const RowScale rs = rowScale(row.Lt);
+            gptr<T> outG = to_global(outRow);
+            unsigned nFlag = 0, nCanc = 0;
+            bool left = false;
+            for (int w0 = 0; w0 < nvRow; w0 += 64) {
+                const int i = w0 + lane;
+                const double den2 = windowDen2(pf[ppad(min(i, N))], pf[ppad(min(i + row.Lt, N))], rs.lt);
+                const float d2 = static_cast<float>(den2);
+                const bool fl = i < nvRow && !(d2 > rs.thr);
+                if (__ballot(fl) == 0ull) { continue; }
+                const bool canc = fl && !(den2 > rs.kc);
+                nFlag += __popcll(__ballot(fl));
+                nCanc += __popcll(__ballot(canc));
+                const bool flat = canc && constant_window(eqw, i, row.Lt);
+                if (flat) { outG[i] = T(0); }
+                const unsigned long long m = __ballot(fl && !flat);
+                if (m == 0ull) { continue; }
+                if constexpr (QUEUE) {
+                    left = true;
+                } else {
+                    T s = T(1);
+                    if (fl && !flat) { s = canc ? scale_exact<T>() : -static_cast<T>(scaleOf(d2, rs.sqrtLt)); }
+                    fixup_chunk<T>(x, s, to_global(row.tmpl), row.Lt, outG, w0, lane, a, m);
+                }
+            }
+            if (lane == 0) { countFlags(nFlag, nCanc); }
+            if (left) { recordRow(rowIdx, 0, nvRow); }
             return;
         }
         T *own = reinterpret_cast<T *>(xb + wave * XW);
@@ -982,14 +1147,23 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
         for (int g0 = sg.rowBegin; g0 < rowEnd;) {
             const int g1 = groupEnd(g0);
             if (g1 - g0 >= kCorr2SharedGroup) {
-                const int myFlags = compute_scale<T, TILE, 1, QUEUE>(raw, ts1, ts2, tp1, tp2, sc, a, nValidSeg,
-                                                                     rows[g0].Lt, noise, tid, NT);
-                const bool anyFlag = __syncthreads_or(myFlags) != 0;
+                // packed counts (flagged + cancelled << 16) and kFix
+                int myFlags;
+                if constexpr (PREFIX) {
+                    myFlags = prefixScale(rows[g0].Lt);
+                } else {
+                    myFlags = compute_scale<T, TILE, 1, QUEUE>(raw, ts1, ts2, tp1, tp2, sc, a, nValidSeg, rows[g0].Lt,
+                                                               noise, tid, NT);
+                    if (myFlags != 0) { myFlags |= kFix; }
+                }
+                // __syncthreads_or gives a truth value, not the bits
+                int any = __syncthreads_or(myFlags);
+                if (any != 0 && __syncthreads_or(myFlags & kFix) != 0) { any |= kFix; }
                 double flagSum = 0;
-                if (QUEUE && anyFlag) { flagSum = uniform(block_sum<NT>(static_cast<double>(myFlags), red)); }
+                if (QUEUE && any != 0) { flagSum = uniform(block_sum<NT>(static_cast<double>(myFlags & ~kFix), red)); }
                 for (int r = g0 + wave; r < g1; r += NWAVE) {
                     startRow(rows[r]);
-                    finishRow(rows[r], r, sc, anyFlag, flagSum);
+                    finishRow(rows[r], r, sc, any, flagSum);
                 }
                 __syncthreads();  // sc is rebuilt for the next group
             }
@@ -1017,7 +1191,7 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
     };
     for (int cur = nextSolo(); cur >= 0; cur = nextSolo()) {
         startRow(rows[cur]);
-        finishRow(rows[cur], cur, nullptr, false, 0.0);
+        finishRow(rows[cur], cur, nullptr, 0, 0.0);
     }
 }
 

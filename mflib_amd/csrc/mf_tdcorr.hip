@@ -51,6 +51,7 @@ constexpr int NT = kThreads;
 constexpr int IS = kTdOutputsPerItem;  // outputs per work item
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
@@ -78,6 +79,13 @@ struct TdTraits<__bf16> {
 };
 
 constexpr int kTdCoopFlags = 4;  // at most this many left at the end: the wave shares each window
+
+// Tiles with at least this many windows whose numerator is recomputed take
+// the whole tile's numerators on FP64 MFMA (16 x 16 windows, 64 products of
+// 64 cycles at 256 taps: 4100 cycles of one SIMD), fewer go one by one to
+// the queue kernel (227 SIMD cycles each, measured: 10.7 M windows of about
+// 190 taps in 0.99 ms): the lines cross at 18.
+constexpr int kTdTileFlags = 20;
 
 // Exact FP64 value of one flagged window at item offset i, over taps
 // m = m0, m0 + step, ... (one lane: 0, 1; a whole wave: lane, 64, summed
@@ -354,6 +362,7 @@ __global__ __launch_bounds__(NT, (td_blocks_per_cu<MT>())) void tdcorr_kernel(co
         int LtR[4], nvR[4];
         float kcR[4], knR[4], slR[4];
         gptr<float> outR[4];
+        int fullOut = IS;  // outputs every row of the group has
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int j = 4 * quad + r;
@@ -363,7 +372,7 @@ __global__ __launch_bounds__(NT, (td_blocks_per_cu<MT>())) void tdcorr_kernel(co
                 nvR[r] = static_cast<int>(max(0ll, min(static_cast<long long>(IS), row.nOut - base)));
                 kcR[r] = row.kc;
                 knR[r] = row.kn;
-                slR[r] = row.sqrtLt;
+                slR[r] = row.sqrtLt * scF;
                 outR[r] = to_global(static_cast<float *>(row.out)) + base;
             } else {
                 LtR[r] = 1;
@@ -373,7 +382,10 @@ __global__ __launch_bounds__(NT, (td_blocks_per_cu<MT>())) void tdcorr_kernel(co
                 slR[r] = 0.0f;
                 outR[r] = nullptr;
             }
+            fullOut = min(fullOut, nvR[r]);
         }
+        fullOut = min(fullOut, __shfl_xor(fullOut, 16, 64));
+        fullOut = __builtin_amdgcn_readfirstlane(min(fullOut, __shfl_xor(fullOut, 32, 64)));
         unsigned tiles = 0;  // tiles with flagged windows (wave-uniform)
         for (int tile = 0; tile < kTdTiles; ++tile) {
             const int i0 = 16 * tile;
@@ -397,37 +409,60 @@ __global__ __launch_bounds__(NT, (td_blocks_per_cu<MT>())) void tdcorr_kernel(co
                     acc1 = Tr::mfma(ap[1][st], b1, acc1);
                 }
             }
-            // epilogue: normalise, flag, store
+            // epilogue: normalise, flag, store.  A window is flagged unless
+            // den2 - kn S2 is above the cancellation floor (kc is far below
+            // kn, so its test is left to the windows this one flags); where
+            // every row has the tile's outputs, flagged ones are stored too
+            // and overwritten later.
             const int i = i0 + c16;
             const double p1i = sm.P1[i], p2i = sm.P2[i];
-            unsigned bits = 0;
+            const bool full = i0 + 16 <= fullOut;  // uniform
+            float rho[4];
+            unsigned long long flags[4], any = 0;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int Lt = LtR[r];
                 // window sums in FP64 (differences of the block's prefix
                 // sums), the rest in FP32
-                const double S1 = sm.P1[i + Lt] - p1i;
-                const double S2 = sm.P2[i + Lt] - p2i;
-                const float d2 = static_cast<float>(fma(-S1, S1, Lt * S2));
-                const float s2 = static_cast<float>(S2);
-                const bool canc = !(d2 > fmaf(kcR[r], s2, flK * static_cast<float>(Lt)));
-                const bool flag = canc || knR[r] * s2 > d2;
+                const double S1 = sm.P1[i + LtR[r]] - p1i;
+                const double S2 = sm.P2[i + LtR[r]] - p2i;
+                const float d2 = static_cast<float>(fma(-S1, S1, LtR[r] * S2));
+                flags[r] = __ballot(!(fmaf(-knR[r], static_cast<float>(S2), d2) > flK * static_cast<float>(LtR[r])));
+                any |= flags[r];
                 float y = __builtin_amdgcn_rsqf(d2);
                 y = y * (1.5f - 0.5f * d2 * y * y);
-                const float rho = (acc0[r] + acc1[r]) * (scF * slR[r] * y);
-                const bool valid = i < nvR[r];
-                if (valid && !flag) { outR[r][i] = rho; }
-                bits |= (valid && flag ? 1u : 0u) << r;
-                bits |= (valid && canc ? 1u : 0u) << (4 + r);
+                rho[r] = (acc0[r] + acc1[r]) * (slR[r] * y);
             }
-            if (__ballot(bits != 0u) != 0ull) {
-                fq[wave][tile][lane] = static_cast<unsigned char>(bits);
-                tiles |= 1u << tile;
+            if (full) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) { outR[r][i] = rho[r]; }
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    if (i < nvR[r]) { outR[r][i] = rho[r]; }
+                }
+            }
+            if (any != 0ull) {
+                unsigned bits = 0;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const bool flag = i < nvR[r] && ((flags[r] >> lane) & 1u);
+                    const double S1 = sm.P1[i + LtR[r]] - p1i;
+                    const double S2 = sm.P2[i + LtR[r]] - p2i;
+                    const float d2 = static_cast<float>(fma(-S1, S1, LtR[r] * S2));
+                    const float floorR = fmaf(kcR[r], static_cast<float>(S2), flK * static_cast<float>(LtR[r]));
+                    bits |= (flag ? 1u : 0u) << r;
+                    bits |= (flag && !(d2 > floorR) ? 1u : 0u) << (4 + r);
+                }
+                if (__ballot(bits != 0u) != 0ull) {
+                    fq[wave][tile][lane] = static_cast<unsigned char>(bits);
+                    tiles |= 1u << tile;
+                }
             }
         }
         // flagged windows of the row group, after its tile loop: exactly
-        // constant windows are 0 at once, the others go to the device
-        // queue (fix_kernel recomputes them after the launch), or, when it
+        // constant windows are 0 at once; a tile of many windows that keep
+        // their norm gets its numerators on FP64 MFMA; the others go to the
+        // device queue (fix_kernel recomputes them after the launch), or, when it
         // is full, to the wave's list, recomputed here one window per lane
         // in passes of 64 (a few left at the end: the whole wave on one
         // window at a time).  List entry: tile (5 bits), step r (2 bits),
@@ -474,6 +509,43 @@ __global__ __launch_bounds__(NT, (td_blocks_per_cu<MT>())) void tdcorr_kernel(co
             }
             nList -= done;
         };
+        // The windows of a tile marked in the low bits of fq: numerators
+        // sum t (x - a) of all 16 x 16 by v_mfma_f64_16x16x4 (row lane % 16
+        // of the taps, column lane % 16 of the Hankel operand, k = lane / 16;
+        // result row 4 r + lane / 16), norms from the FP64 prefix sums.
+        auto exactTile = [&](int tile) {
+            const int i = 16 * tile + c16;
+            const TdRow mine = rows[rowBase + min(c16, nMine - 1)];
+            const gptr<const double> t = to_global(mine.tmpl);
+            const int LtA = c16 < nMine ? mine.Lt : 0;
+            int LtMax = max(max(LtR[0], LtR[1]), max(LtR[2], LtR[3]));
+            LtMax = max(LtMax, __shfl_xor(LtMax, 16, 64));
+            LtMax = __builtin_amdgcn_readfirstlane(max(LtMax, __shfl_xor(LtMax, 32, 64)));
+            f64x4 acc = {};
+            for (int k0 = 0; k0 < LtMax; k0 += 16) {  // LtMax <= KT, a multiple of 16
+                double tk[4], dk[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int k = k0 + 4 * u + quad;
+                    tk[u] = k < LtA ? t[k] : 0.0;
+                    dk[u] = static_cast<double>(sm.raw[i + k]) - a;
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) { acc = __builtin_amdgcn_mfma_f64_16x16x4f64(tk[u], dk[u], acc, 0, 0, 0); }
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                // row 4 r + quad of the result; its mark is bit quad of lane 16 r + c16
+                if ((fq[wave][tile][16 * r + c16] >> quad) & 1u) {
+                    const TdRow row = rows[rowBase + 4 * r + quad];
+                    const double S1 = sm.P1[i + row.Lt] - sm.P1[i];
+                    const double den2 = row.Lt * (sm.P2[i + row.Lt] - sm.P2[i]) - S1 * S1;
+                    double rho = acc[r] * sqrt(row.Lt / den2);
+                    if (fabs(rho) > 1.1) { rho = 0; }
+                    to_global(static_cast<float *>(row.out))[base + i] = static_cast<float>(rho);
+                }
+            }
+        };
         while (tiles != 0u) {
             const int tile = __ffs(tiles) - 1;
             tiles &= tiles - 1u;
@@ -481,14 +553,11 @@ __global__ __launch_bounds__(NT, (td_blocks_per_cu<MT>())) void tdcorr_kernel(co
             const unsigned word = fq[wave][tile][lane];
             const unsigned flg = word & 15u;
             const unsigned cnc = word >> 4;
-            int total = __popc(flg), full = __popc(flg & cnc);
 #pragma unroll
-            for (int o = 32; o > 0; o >>= 1) {
-                total += __shfl_xor(total, o, 64);
-                full += __shfl_xor(full, o, 64);
+            for (int r = 0; r < 4; ++r) {
+                nFlag += static_cast<unsigned>(__popcll(__ballot((flg >> r) & 1u)));
+                nCanc += static_cast<unsigned>(__popcll(__ballot(((flg & cnc) >> r) & 1u)));
             }
-            nFlag += static_cast<unsigned long long>(__builtin_amdgcn_readfirstlane(total));
-            nCanc += static_cast<unsigned long long>(__builtin_amdgcn_readfirstlane(full));
             unsigned keep = flg;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -499,9 +568,20 @@ __global__ __launch_bounds__(NT, (td_blocks_per_cu<MT>())) void tdcorr_kernel(co
                     }
                 }
             }
-            int n = 0;
+            const unsigned noisy = keep & ~cnc;
+            int n = 0, nNoisy = 0;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) { n += __popcll(__ballot((keep >> r) & 1u)); }
+            for (int r = 0; r < 4; ++r) {
+                n += __popcll(__ballot((keep >> r) & 1u));
+                nNoisy += __popcll(__ballot((noisy >> r) & 1u));
+            }
+            if (nNoisy >= kTdTileFlags) {
+                fq[wave][tile][lane] = static_cast<unsigned char>(noisy);
+                wave_lds_sync();
+                exactTile(tile);
+                keep &= cnc;
+                n -= nNoisy;
+            }
             if (n == 0) { continue; }
             unsigned long long q0 = 0;
             if (lane == 0) { q0 = atomicAdd(queue.count, static_cast<unsigned long long>(n)); }

@@ -22,7 +22,7 @@
 // tmpl_kernel  -- template demean/normalise and spectrum, FP64.
 // stack_kernel -- moveout-shifted weighted stack of one group.
 // peak_kernel  -- threshold + local-maximum candidates.
-// minmax_kernel -- per-block min/max for the dead-trace test.
+// copy_minmax_kernel -- a signal's copy and its min/max for the dead-trace test.
 #include "mf_device.hpp"
 #include "mf_kernels.hpp"
 #include <cfloat>
@@ -1698,24 +1698,40 @@ __global__ __launch_bounds__(NT) void pack_candidates_kernel(const StackGroup *_
     }
 }
 
+// Copies a signal and takes its minimum and maximum on the way: block b's go
+// to part[2 b] and part[2 b + 1], host memory that the caller reads after the
+// stream has finished.  Whole 16-byte vectors when both sides are aligned.
 template <typename T>
-__global__ __launch_bounds__(NT) void minmax_kernel(const T *__restrict__ x, long long n,
-                                                    double *__restrict__ pmin,
-                                                    double *__restrict__ pmax)
+__global__ __launch_bounds__(NT) void copy_minmax_kernel(const T *src, T *dst, long long n, double *part)
 {
+    constexpr int VEC = 16 / static_cast<int>(sizeof(T));
+    using V = T __attribute__((ext_vector_type(VEC)));
     __shared__ double red[NT / 64];
+    const long long first = static_cast<long long>(blockIdx.x) * NT + threadIdx.x;
     const long long stride = static_cast<long long>(gridDim.x) * NT;
     double lo = DBL_MAX, hi = -DBL_MAX;
-    for (long long i = static_cast<long long>(blockIdx.x) * NT + threadIdx.x; i < n; i += stride) {
-        const double v = static_cast<double>(x[i]);
-        lo = fmin(lo, v);
-        hi = fmax(hi, v);
+    const auto take = [&](T x) {
+        lo = fmin(lo, static_cast<double>(x));
+        hi = fmax(hi, static_cast<double>(x));
+    };
+    const bool aligned = ((reinterpret_cast<unsigned long long>(src) | reinterpret_cast<unsigned long long>(dst)) & 15) == 0;
+    const long long nVec = aligned ? n / VEC : 0;
+    for (long long k = first; k < nVec; k += stride) {
+        const V v = reinterpret_cast<const V *>(src)[k];
+        reinterpret_cast<V *>(dst)[k] = v;
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) { take(v[e]); }
+    }
+    for (long long i = nVec * VEC + first; i < n; i += stride) {
+        const T x = src[i];
+        dst[i] = x;
+        take(x);
     }
     const double bmax = block_max<NT>(hi, red);
     const double bmin = -block_max<NT>(-lo, red);
     if (threadIdx.x == 0) {
-        pmin[blockIdx.x] = bmin;
-        pmax[blockIdx.x] = bmax;
+        part[2 * blockIdx.x] = bmin;
+        part[2 * blockIdx.x + 1] = bmax;
     }
 }
 
@@ -2180,15 +2196,16 @@ hipError_t launch_peaks(int precision, const void *dx, long long n, double thres
     return hipGetLastError();
 }
 
-hipError_t launch_minmax(int precision, const void *dx, long long n, double *dPartMin,
-                         double *dPartMax, int nBlocks, hipStream_t stream)
+hipError_t launch_copy_minmax(int precision, const void *dSrc, void *dDst, long long n, double *part, int nBlocks,
+                              hipStream_t stream)
 {
+    if (n <= 0 || nBlocks <= 0) { return hipErrorInvalidValue; }
     if (precision == 0) {
-        hipLaunchKernelGGL(minmax_kernel<float>, dim3(nBlocks), dim3(NT), 0, stream,
-                           static_cast<const float *>(dx), n, dPartMin, dPartMax);
+        hipLaunchKernelGGL(copy_minmax_kernel<float>, dim3(nBlocks), dim3(NT), 0, stream,
+                           static_cast<const float *>(dSrc), static_cast<float *>(dDst), n, part);
     } else {
-        hipLaunchKernelGGL(minmax_kernel<double>, dim3(nBlocks), dim3(NT), 0, stream,
-                           static_cast<const double *>(dx), n, dPartMin, dPartMax);
+        hipLaunchKernelGGL(copy_minmax_kernel<double>, dim3(nBlocks), dim3(NT), 0, stream,
+                           static_cast<const double *>(dSrc), static_cast<double *>(dDst), n, part);
     }
     return hipGetLastError();
 }

@@ -60,12 +60,15 @@ struct FixQueue {
     unsigned long long *count;
     int *entries;  // 8 bytes per entry
     unsigned long long cap;
-    // row blocks whose flagged windows did not fit the queue: (row, first
-    // output, outputs) per record, recomputed whole; sized by the host for
-    // every row block of the launches (two records per row block at most),
-    // so it cannot overflow.  Only the FFT wave-kernel queue has them.
+    // Records for a launch of their own, overCap of them.  FFT wave kernel:
+    // row blocks with flagged windows (row, first output, outputs), sized by
+    // the host for every row block of the launches (two records per row block
+    // at most), so they cannot overflow.  Time-domain kernel: tiles of many
+    // flagged windows (first row, rows, first output); past overCap a tile is
+    // recomputed in place.
     unsigned long long *overCount;
     int *over;  // 4 ints per record
+    unsigned long long overCap;
 };
 
 // One work item: block `block` of lane `seg`, for the first nRows rows of
@@ -154,7 +157,7 @@ struct TdRow {
 };
 
 // One work item: outputs [seg0, seg0 + kTdOutputsPerItem) of lane `seg`
-// for rows [rowBegin, rowBegin + nRows) (nRows <= 128) of the row table.
+// for rows [rowBegin, rowBegin + nRows) of the row table.
 struct TdItem {
     int seg;
     int rowBegin;
@@ -180,6 +183,7 @@ hipError_t launch_td(int kind, int KT, const TdItem *dItems, int nItems, const S
 // launches that filled the queue), for either row table
 hipError_t launch_fix(const Row *dRows, FixQueue queue, int blocks, hipStream_t stream);  // and its overflow records
 hipError_t launch_fix(const TdRow *dRows, FixQueue queue, int blocks, hipStream_t stream);
+hipError_t launch_fix_tiles(const TdRow *dRows, FixQueue queue, int blocks, hipStream_t stream);
 
 // Correlation + normalisation: one launch per FFT size.  Variant 1 runs
 // block-wide LDS Stockham FFTs; variant 2 runs wave-level register FFTs
@@ -241,9 +245,11 @@ hipError_t launch_peaks(int precision, const void *dx, long long n, double thres
 // channel.  dPart holds 2 * nSegs * ceil(maxN / kDeadChunk) doubles.
 hipError_t launch_seg_dead(int precision, Seg *dSegs, int nSegs, long long maxN, double *dPart,
                            hipStream_t stream);
-// Per-block min and max of a signal (dead-trace test on device input).
-hipError_t launch_minmax(int precision, const void *dx, long long n, double *dPartMin,
-                         double *dPartMax, int nBlocks, hipStream_t stream);
+// Copies n samples and writes each block's min and max to part[2 b],
+// part[2 b + 1] (memory the device can write, such as pinned host memory):
+// the dead-trace test of a signal handed over in device memory.
+hipError_t launch_copy_minmax(int precision, const void *dSrc, void *dDst, long long n, double *part, int nBlocks,
+                              hipStream_t stream);
 
 // Window scales sqrt(Lt)/sqrt(Lt S2 - S1^2) of the n - Lt + 1 windows of a
 // FP32 signal from prefix scans: FP64 scans (kScanF64) or compensated

@@ -18,12 +18,12 @@
 // rho = s * D * scale with the window normalisation from FP64 prefix sums
 // of the block.
 //
-// Work item: IS = 512 consecutive outputs of the lane and up to 128 rows.
+// Work item: IS = 512 consecutive outputs of the lane and up to 192 rows.
 // Each of the 4 waves takes 16 rows at a time: their split taps stay in
 // registers (weight-stationary, parts * KT / 8 VGPRs) while the wave walks
-// the 32 output tiles of 16; the Hankel operand is read from LDS, where
-// entry p holds the 8 samples x~[p .. p+7] (one 16-byte read per part and
-// k-step of 32).
+// the 32 output tiles of 16; the Hankel operand's entry p, the 8 samples
+// x~[p .. p+7], is read from LDS for one k-step of 32 per tile and part and
+// stays in a ring of registers.
 //
 // Accuracy: per window |d rho| <= eps_m * sqrt(Lt S2) / den with
 // eps_m = eps_split + (4 sqrt(KT/16) + 4) 2^-24 (FP32 accumulation over at
@@ -87,6 +87,11 @@ constexpr int kTdCoopFlags = 4;  // at most this many left at the end: the wave 
 // 190 taps in 0.99 ms): the lines cross at 18.
 constexpr int kTdTileFlags = 20;
 
+// FP64 prefix sums of d = x - a and of d^2 at one sample.
+struct __align__(16) TdSums {
+    double s1, s2;
+};
+
 // Exact FP64 value of one flagged window at item offset i, over taps
 // m = m0, m0 + step, ... (one lane: 0, 1; a whole wave: lane, 64, summed
 // across the wave).
@@ -98,7 +103,7 @@ constexpr int kTdTileFlags = 20;
 //  - noise flag: the numerator sum t (x - a) from the anchored samples with
 //    the window norm from the block's FP64 prefix sums, accurate there.
 // |rho| > 1.1 gives 0 (the reference's tooBig rule).
-__device__ double exact_window_td(const float *raw, const double *P1, const double *P2, int i,
+__device__ double exact_window_td(const float *raw, const TdSums *P, int i,
                                   gptr<const double> t, int Lt, double a, bool canc, int m0, int step)
 {
     const double shift = canc ? static_cast<double>(raw[i]) : a;
@@ -119,8 +124,8 @@ __device__ double exact_window_td(const float *raw, const double *P1, const doub
     if (canc) {
         rho = dn / fmax(DBL_EPSILON, sqrt(fmax(0.0, s2 - s1 * s1 / Lt)));
     } else {
-        const double S1 = P1[i + Lt] - P1[i];
-        const double den2 = Lt * (P2[i + Lt] - P2[i]) - S1 * S1;
+        const double S1 = P[i + Lt].s1 - P[i].s1;
+        const double den2 = Lt * (P[i + Lt].s2 - P[i].s2) - S1 * S1;
         rho = dn * sqrt(Lt / den2);
     }
     return fabs(rho) > 1.1 ? 0.0 : rho;
@@ -131,13 +136,16 @@ template <typename MT, int KT>
 struct TdStage {
     static constexpr int NP = TdTraits<MT>::parts;
     static constexpr int SPAN = IS + KT;  // samples one item reads
-    MT x8[NP][SPAN][8];                   // entry p of part q: x~[p .. p+7]
+    // x~ of each part as pairs of samples in two copies: pair w of copy c is
+    // samples 2 w + c and 2 w + c + 1, so the 8 samples from p on are four
+    // consecutive words of copy p mod 2
+    unsigned x2[NP][2][SPAN / 2];
     float raw[SPAN];                      // samples (FP32), for exact windows
-    double P1[SPAN + 1];                  // prefix sums of d = x - a
-    double P2[SPAN + 1];                  //   and of d^2
-    double red[NT / 64];
-    double wsum1[NT / 64], wsum2[NT / 64];
-    unsigned eqw[(SPAN + 31) / 32];       // bit p: sample p equals sample p + 1 (constant windows)
+    TdSums P[SPAN + 1];                   // prefix sums
+    double tot1[NT / 64], tot2[NT / 64];
+    unsigned eqw[(SPAN + 31) / 32];       // bit p: sample p equals sample p + 1
+    unsigned short run[SPAN];             // set bits from bit p on, up to 256 (blocks with any):
+                                          // the window at p is constant when run[p] >= Lt - 1
 };
 
 // What the epilogue needs of the staged block: the anchor a, the scale s
@@ -146,12 +154,17 @@ struct TdBlock {
     double a;
     float scF;
     float flK;
+    bool equal;  // some sample equals its neighbour: `run` is filled
 };
 
 // Stages outputs [base, base + IS) of lane sg: loads the samples, takes the
-// block anchor and RMS, splits x~ into the 8-wide Hankel entries of every
-// part, builds the FP64 prefix sums and the equal-neighbour bits.  The
-// caller synchronises the block before reading any of it.
+// anchor (the mean of 64 samples spread over the block, taken by every wave:
+// any value near the samples will do) and the RMS about it, splits x~ into
+// its parts, builds the FP64 prefix sums and the equal-neighbour bits.  Each
+// thread takes consecutive samples and the scan runs on DPP moves, with one
+// barrier inside (the split by LDS copies of every entry, sums behind four
+// barriers and bits on one wave took 20 % of the kernel).  Ends with the
+// block synchronised.
 template <typename MT, int KT>
 __device__ __forceinline__ TdBlock td_stage(TdStage<MT, KT> &sm, const Seg &sg, long long base)
 {
@@ -161,105 +174,104 @@ __device__ __forceinline__ TdBlock td_stage(TdStage<MT, KT> &sm, const Seg &sg, 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;
-    // 1. samples, anchor and scale
-    const gptr<const float> x = to_global(static_cast<const float *>(sg.x));
+    // 1. samples, anchor, running sums
+    const gptr<const float> x = to_global(static_cast<const float *>(sg.x)) + base;
     const int nSamp = static_cast<int>(min(static_cast<long long>(SPAN), sg.n - base));
+    const float spread = x[min(lane * (SPAN / 64), nSamp - 1)];
+    const int p0 = tid * SPT;
     float v[SPT];
-    double s = 0;
+#pragma unroll
+    for (int q = 0; q < SPT; ++q) { v[q] = p0 + q < nSamp ? x[p0 + q] : 0.0f; }
+    const float after = p0 + SPT < nSamp ? x[p0 + SPT] : 0.0f;
+    if (tid < (SPAN + 31) / 32) { sm.eqw[tid] = 0u; }
+    const double a = static_cast<double>(read_lane(wave_scan_sum(spread * (1.0f / 64)), 63));
+    double t1 = 0, t2 = 0;
+    double l1[SPT], l2[SPT];  // exclusive sums inside the thread
 #pragma unroll
     for (int q = 0; q < SPT; ++q) {
-        const int p = tid * SPT + q;  // contiguous run per thread (for the scan)
-        const float val = (p < nSamp) ? x[base + p] : 0.0f;
-        v[q] = val;
-        if (p < SPAN) { sm.raw[p] = val; }
-        s += static_cast<double>(val);
+        const double d = p0 + q < nSamp ? static_cast<double>(v[q]) - a : 0.0;
+        l1[q] = t1;
+        l2[q] = t2;
+        t1 += d;
+        t2 += d * d;
+        if (p0 + q < SPAN) { sm.raw[p0 + q] = v[q]; }
     }
-    const double a = block_sum<NT>(s, sm.red) / nSamp;
-    double e = 0, l1 = 0, l2 = 0;
-    double d1[SPT], d2[SPT];
+    const double i1 = wave_scan_sum(t1), i2 = wave_scan_sum(t2);
+    if (lane == 63) {
+        sm.tot1[wave] = i1;
+        sm.tot2[wave] = i2;
+    }
+    __syncthreads();
+    double energy = 0, o1 = 0, o2 = 0;
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) {
+        if (w == wave) {
+            o1 += i1 - t1;
+            o2 = energy + (i2 - t2);
+        } else if (w < wave) {
+            o1 += sm.tot1[w];
+        }
+        energy += sm.tot2[w];
+    }
+    // 2. prefix sums P[p] = sum over q < p, equal-neighbour bits
+    int equal = 0;
 #pragma unroll
     for (int q = 0; q < SPT; ++q) {
-        const int p = tid * SPT + q;
-        const double d = (p < nSamp) ? static_cast<double>(v[q]) - a : 0.0;
-        d1[q] = l1;  // exclusive local prefix
-        d2[q] = l2;
-        l1 += d;
-        l2 += d * d;
-        e += d * d;
+        if (p0 + q < SPAN) { sm.P[p0 + q] = TdSums{o1 + l1[q], o2 + l2[q]}; }
+        if (p0 + q == SPAN - 1) {
+            const double d = p0 + q < nSamp ? static_cast<double>(v[q]) - a : 0.0;
+            sm.P[SPAN] = TdSums{o1 + l1[q] + d, o2 + l2[q] + d * d};
+        }
+        const float next = q + 1 < SPT ? v[q + 1 < SPT ? q + 1 : q] : after;
+        if (p0 + q + 1 < SPAN && v[q] == next) {
+            atomicOr(&sm.eqw[(p0 + q) >> 5], 1u << ((p0 + q) & 31));
+            equal = 1;
+        }
     }
-    const double energy = block_sum<NT>(e, sm.red);
+    // 3. the parts of x~ = (x - a) / sc.  The FP32 value is the sum of its
+    //    parts exactly (each remainder is exact in FP32 and the parts
+    //    together hold at least 24 significant bits).
     const double sc = energy > 0 ? sqrt(energy / nSamp) : 1.0;
     const float inv = static_cast<float>(1.0 / sc);
-    // 2. split samples into the 8-wide Hankel entries: sample p goes to
-    //    entry p - k, slot k (k = 0..7), of every part.  The FP32 value
-    //    xs is the sum of its parts exactly (each remainder is exact in
-    //    FP32 and the parts together hold at least 24 significant bits).
 #pragma unroll
     for (int q = 0; q < SPT; ++q) {
-        const int p = tid * SPT + q;
+        const int p = p0 + q;
         if (p < SPAN) {
-            float rest = (p < nSamp) ? static_cast<float>((static_cast<double>(v[q]) - a) * inv) : 0.0f;
+            float rest = p < nSamp ? static_cast<float>((static_cast<double>(v[q]) - a) * inv) : 0.0f;
 #pragma unroll
             for (int pt = 0; pt < NP; ++pt) {
                 const MT part = static_cast<MT>(rest);
                 rest -= static_cast<float>(part);
-#pragma unroll
-                for (int k = 0; k < 8; ++k) {
-                    if (p - k >= 0) { sm.x8[pt][p - k][k] = part; }
-                }
+                reinterpret_cast<MT *>(sm.x2[pt][0])[p] = part;
+                if (p > 0) { reinterpret_cast<MT *>(sm.x2[pt][1])[p - 1] = part; }
+                if (p == SPAN - 1) { reinterpret_cast<MT *>(sm.x2[pt][1])[p] = static_cast<MT>(0.0f); }
             }
         }
     }
-    // entries past the span read zeros in their upper slots
-    for (int p = SPAN - 7 + tid; p < SPAN; p += NT) {
-        for (int k = SPAN - p; k < 8; ++k) {
+    const bool any = __syncthreads_or(equal) != 0;
+    if (any) {  // 4. run lengths of the bits
+        constexpr int W = (SPAN + 31) / 32;
+        int run = 0;
+        for (int p = p0 + SPT; run < 256 && p < SPAN;) {  // of the next thread's first sample
+            const unsigned rest = sm.eqw[p >> 5] >> (p & 31);
+            const int take = min(32 - (p & 31), SPAN - p);
+            const int ones = min(rest == ~0u ? 32 : __ffs(~rest) - 1, take);
+            run += ones;
+            if (ones < take) { break; }
+            p += take;
+        }
+        static_assert(W * 32 >= SPAN, "words");
 #pragma unroll
-            for (int pt = 0; pt < NP; ++pt) { sm.x8[pt][p][k] = static_cast<MT>(0.0f); }
+        for (int q = SPT - 1; q >= 0; --q) {
+            const int p = p0 + q;
+            if (p < SPAN) {
+                run = (sm.eqw[p >> 5] >> (p & 31)) & 1u ? min(run + 1, 256) : 0;
+                sm.run[p] = static_cast<unsigned short>(run);
+            }
         }
+        __syncthreads();
     }
-    // 3. FP64 prefix sums P[p] = sum_{q < p} d_q (thread runs, then waves)
-    double x1 = l1, x2 = l2;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const double y1 = __shfl_up(x1, o, 64);
-        const double y2 = __shfl_up(x2, o, 64);
-        if (lane >= o) {
-            x1 += y1;
-            x2 += y2;
-        }
-    }
-    if (lane == 63) {
-        sm.wsum1[wave] = x1;
-        sm.wsum2[wave] = x2;
-    }
-    __syncthreads();
-    if (tid < (SPAN + 31) / 32) {
-        unsigned bits = 0;
-        for (int b = 0; b < 32; ++b) {
-            const int p = 32 * tid + b;
-            if (p + 1 < SPAN && sm.raw[p] == sm.raw[p + 1]) { bits |= 1u << b; }
-        }
-        sm.eqw[tid] = bits;
-    }
-    double w1 = 0, w2 = 0;
-    for (int w = 0; w < wave; ++w) {
-        w1 += sm.wsum1[w];
-        w2 += sm.wsum2[w];
-    }
-    const double e1 = w1 + x1 - l1, e2 = w2 + x2 - l2;  // exclusive prefix of this thread's run
-#pragma unroll
-    for (int q = 0; q < SPT; ++q) {
-        const int p = tid * SPT + q;
-        if (p < SPAN) {
-            sm.P1[p] = e1 + d1[q];
-            sm.P2[p] = e2 + d2[q];
-        }
-    }
-    if (tid == NT - 1) {
-        sm.P1[SPAN] = w1 + x1;
-        sm.P2[SPAN] = w2 + x2;
-    }
-    return TdBlock{a, static_cast<float>(sc), static_cast<float>(1.0e-12 * energy)};
+    return TdBlock{a, static_cast<float>(sc), static_cast<float>(1.0e-12 * energy), any};
 }
 
 // A dead lane's item: zeros in every row.
@@ -283,23 +295,24 @@ __device__ __forceinline__ void td_dead(const TdItem &item, const TdRow *__restr
 // constants stay in registers for the row group, and each quarter wave
 // stores 16 consecutive outputs of its row.
 constexpr int kTdTiles = IS / 16;        // output tiles of 16 per item
+constexpr int kTdRingParts = 2;          // operand parts whose steps stay in registers
 constexpr int kTdFixList = 64 + 4 * 64;  // carried over plus one tile's windows
 
-// Blocks per CU the register budget is capped for: three for the FP16 pair
-// (64 VGPRs of taps at KT = 256, 51 KB of LDS per block), two for the BF16
-// triple (96 VGPRs of taps, 63 KB of LDS).
-template <typename MT>
-constexpr int td_blocks_per_cu() { return TdTraits<MT>::parts == 2 ? 3 : 2; }
+// Blocks per CU the register budget is capped for: two, at KT = 256 64 (FP16
+// pair) or 96 (BF16 triple) registers of taps and 64 of the operand ring.
+constexpr int kTdBlocks = 2;
 
 template <typename MT, int KT>
-__global__ __launch_bounds__(NT, (td_blocks_per_cu<MT>())) void tdcorr_kernel(const TdItem *__restrict__ items,
+__global__ __launch_bounds__(NT, kTdBlocks) void tdcorr_kernel(const TdItem *__restrict__ items,
                                                        const Seg *__restrict__ segs,
                                                        const TdRow *__restrict__ rows, FixQueue queue)
 {
     using Tr = TdTraits<MT>;
     using V8 = typename Tr::vec8;
+    typedef int WordsU __attribute__((ext_vector_type(4), aligned(4)));  // four words at any word
     constexpr int NP = Tr::parts;
     constexpr int NS = KT / 32;  // k-steps of 32
+    constexpr int RP = kTdRingParts;
     __shared__ __align__(16) TdStage<MT, KT> sm;
     // flagged windows of each wave's tiles: bit r flags the lane's window
     // r, bit 4 + r marks a cancelled variance
@@ -331,7 +344,6 @@ __global__ __launch_bounds__(NT, (td_blocks_per_cu<MT>())) void tdcorr_kernel(co
     const double a = blk.a;
     const float scF = blk.scF;
     const float flK = blk.flK;
-    __syncthreads();  // Hankel entries, prefix sums and raw samples ready
 
     unsigned long long nFlag = 0, nCanc = 0;  // windows recomputed by this wave, in full
     for (int g = 0; 64 * g < item.nRows; ++g) {
@@ -387,82 +399,120 @@ __global__ __launch_bounds__(NT, (td_blocks_per_cu<MT>())) void tdcorr_kernel(co
         fullOut = min(fullOut, __shfl_xor(fullOut, 16, 64));
         fullOut = __builtin_amdgcn_readfirstlane(min(fullOut, __shfl_xor(fullOut, 32, 64)));
         unsigned tiles = 0;  // tiles with flagged windows (wave-uniform)
-        for (int tile = 0; tile < kTdTiles; ++tile) {
-            const int i0 = 16 * tile;
-            f32x4 acc0 = {}, acc1 = {};
-            // B operand: column i0 + c16, taps 32 s + 8 kq + 0..7 = entry
-            // i0 + c16 + 8 kq + 32 s
-            const i32x4 *b0p = reinterpret_cast<const i32x4 *>(&sm.x8[0][i0 + c16 + 8 * kq][0]);
-            const i32x4 *b1p = reinterpret_cast<const i32x4 *>(&sm.x8[1][i0 + c16 + 8 * kq][0]);
-            const i32x4 *b2p = reinterpret_cast<const i32x4 *>(&sm.x8[NP - 1][i0 + c16 + 8 * kq][0]);
+        // B operand: column i0 + c16, taps 32 st + 8 kq + 0..7 = entry
+        // i0 + c16 + 8 kq + 32 st.  Step st of the tile 32 outputs on is this
+        // tile's step st + 1, so the wave walks the even tiles, then the odd
+        // ones, with its steps in a ring of registers and reads one new step
+        // per tile.  (With every step read for every tile the LDS pipe, shared
+        // by the four SIMDs, set the time: 168 of its cycles per tile against
+        // 384 / 4 of the matrix cores.)  The ring turns with the unrolled
+        // tiles, so its slots are compile-time.
+        for (int par = 0; par < 2; ++par) {
+            const int e0 = 16 * par + c16 + 8 * kq;
+            const auto entry = [&](int pt, int step) {
+                return __builtin_bit_cast(V8, *reinterpret_cast<const WordsU *>(&sm.x2[pt][e0 & 1][(e0 >> 1) + 16 * step]));
+            };
+            V8 ring[RP][NS];
 #pragma unroll
-            for (int st = 0; st < NS; ++st) {
-                const V8 b0 = __builtin_bit_cast(V8, b0p[32 * st]);
-                const V8 b1 = __builtin_bit_cast(V8, b1p[32 * st]);
-                acc0 = Tr::mfma(ap[0][st], b0, acc0);
-                acc1 = Tr::mfma(ap[0][st], b1, acc1);
-                acc1 = Tr::mfma(ap[1][st], b0, acc1);
-                if constexpr (NP == 3) {
-                    const V8 b2 = __builtin_bit_cast(V8, b2p[32 * st]);
-                    acc1 = Tr::mfma(ap[0][st], b2, acc1);
-                    acc1 = Tr::mfma(ap[NP - 1][st], b0, acc1);
-                    acc1 = Tr::mfma(ap[1][st], b1, acc1);
-                }
+            for (int pt = 0; pt < RP; ++pt) {
+#pragma unroll
+                for (int st = 0; st < NS; ++st) { ring[pt][st] = entry(pt, st); }
             }
-            // epilogue: normalise, flag, store.  A window is flagged unless
-            // den2 - kn S2 is above the cancellation floor (kc is far below
-            // kn, so its test is left to the windows this one flags); where
-            // every row has the tile's outputs, flagged ones are stored too
-            // and overwritten later.
-            const int i = i0 + c16;
-            const double p1i = sm.P1[i], p2i = sm.P2[i];
-            const bool full = i0 + 16 <= fullOut;  // uniform
-            float rho[4];
-            unsigned long long flags[4], any = 0;
+            for (int t0 = 0; t0 < kTdTiles / 2; t0 += NS) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                // window sums in FP64 (differences of the block's prefix
-                // sums), the rest in FP32
-                const double S1 = sm.P1[i + LtR[r]] - p1i;
-                const double S2 = sm.P2[i + LtR[r]] - p2i;
-                const float d2 = static_cast<float>(fma(-S1, S1, LtR[r] * S2));
-                flags[r] = __ballot(!(fmaf(-knR[r], static_cast<float>(S2), d2) > flK * static_cast<float>(LtR[r])));
-                any |= flags[r];
-                float y = __builtin_amdgcn_rsqf(d2);
-                y = y * (1.5f - 0.5f * d2 * y * y);
-                rho[r] = (acc0[r] + acc1[r]) * (slR[r] * y);
-            }
-            if (full) {
+                for (int u = 0; u < NS; ++u) {
+                    const int t = t0 + u;
+                    const int tile = 2 * t + par;
+                    const int i0 = 16 * tile;
+                    f32x4 acc0 = {}, acc1 = {}, acc2 = {};
 #pragma unroll
-                for (int r = 0; r < 4; ++r) { outR[r][i] = rho[r]; }
-            } else {
+                    for (int st = 0; st < NS; ++st) {
+                        const V8 b0 = ring[0][(u + st) % NS], b1 = ring[1][(u + st) % NS];
+                        acc0 = Tr::mfma(ap[0][st], b0, acc0);
+                        acc1 = Tr::mfma(ap[0][st], b1, acc1);
+                        acc2 = Tr::mfma(ap[1][st], b0, acc2);
+                        if constexpr (NP == 3) {
+                            const V8 b2 = entry(NP - 1, t + st);  // the BF16 triple's third part
+                            acc1 = Tr::mfma(ap[0][st], b2, acc1);
+                            acc2 = Tr::mfma(ap[NP - 1][st], b0, acc2);
+                            acc1 = Tr::mfma(ap[1][st], b1, acc1);
+                        }
+                    }
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    if (i < nvR[r]) { outR[r][i] = rho[r]; }
-                }
-            }
-            if (any != 0ull) {
-                unsigned bits = 0;
+                    for (int r = 0; r < 4; ++r) { acc1[r] += acc2[r]; }
+                    // the next tile's last step (the last tile reads its own again)
+                    const int next = min(t + 1, kTdTiles / 2 - 1) + NS - 1;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const bool flag = i < nvR[r] && ((flags[r] >> lane) & 1u);
-                    const double S1 = sm.P1[i + LtR[r]] - p1i;
-                    const double S2 = sm.P2[i + LtR[r]] - p2i;
-                    const float d2 = static_cast<float>(fma(-S1, S1, LtR[r] * S2));
-                    const float floorR = fmaf(kcR[r], static_cast<float>(S2), flK * static_cast<float>(LtR[r]));
-                    bits |= (flag ? 1u : 0u) << r;
-                    bits |= (flag && !(d2 > floorR) ? 1u : 0u) << (4 + r);
-                }
-                if (__ballot(bits != 0u) != 0ull) {
-                    fq[wave][tile][lane] = static_cast<unsigned char>(bits);
-                    tiles |= 1u << tile;
+                    for (int pt = 0; pt < RP; ++pt) { ring[pt][u] = entry(pt, next); }
+                    // epilogue: normalise, flag, store.  A window is flagged unless
+                    // den2 - kn S2 is above the cancellation floor (kc is far below
+                    // kn, so its test is left to the windows this one flags); where
+                    // every row has the tile's outputs, flagged ones are stored too
+                    // and overwritten later.
+                    const int i = i0 + c16;
+                    const TdSums pi = sm.P[i];
+                    const bool full = i0 + 16 <= fullOut;  // uniform
+                    float rho[4];
+                    unsigned long long flags[4], any = 0;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        // window sums in FP64 (differences of the block's prefix
+                        // sums), the rest in FP32
+                        const TdSums pe = sm.P[i + LtR[r]];
+                        const double S1 = pe.s1 - pi.s1, S2 = pe.s2 - pi.s2;
+                        const float d2 = static_cast<float>(fma(-S1, S1, LtR[r] * S2));
+                        flags[r] = __ballot(!(fmaf(-knR[r], static_cast<float>(S2), d2) > flK * static_cast<float>(LtR[r])));
+                        any |= flags[r];
+                        float y = __builtin_amdgcn_rsqf(d2);
+                        y = y * (1.5f - 0.5f * d2 * y * y);
+                        rho[r] = (acc0[r] + acc1[r]) * (slR[r] * y);
+                    }
+                    if (full) {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) { outR[r][i] = rho[r]; }
+                    } else {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            if (i < nvR[r]) { outR[r][i] = rho[r]; }
+                        }
+                    }
+                    if (any != 0ull) {
+                        // exactly constant windows (a gap's) are 0 at once; the rest
+                        // wait for the end of the row group
+                        const int run = blk.equal ? sm.run[i] : 0;
+                        unsigned bits = 0;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const bool flag = i < nvR[r] && ((flags[r] >> lane) & 1u);
+                            const bool flat = flag && run > 0 && run >= LtR[r] - 1;
+                            if (flat) { outR[r][i] = 0.0f; }
+                            const unsigned nFlat = static_cast<unsigned>(__popcll(__ballot(flat)));
+                            nFlag += nFlat;
+                            nCanc += nFlat;
+                            bits |= (flag && !flat ? 1u : 0u) << r;
+                        }
+                        if (__ballot(bits != 0u) != 0ull) {
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) {
+                                const TdSums pe = sm.P[i + LtR[r]];
+                                const double S1 = pe.s1 - pi.s1, S2 = pe.s2 - pi.s2;
+                                const float d2 = static_cast<float>(fma(-S1, S1, LtR[r] * S2));
+                                const float floorR = fmaf(kcR[r], static_cast<float>(S2), flK * static_cast<float>(LtR[r]));
+                                bits |= (((bits >> r) & 1u) && !(d2 > floorR) ? 1u : 0u) << (4 + r);
+                            }
+                        }
+                        if (__ballot(bits != 0u) != 0ull) {
+                            fq[wave][tile][lane] = static_cast<unsigned char>(bits);
+                            tiles |= 1u << tile;
+                        }
+                    }
                 }
             }
         }
-        // flagged windows of the row group, after its tile loop: exactly
-        // constant windows are 0 at once; a tile of many windows that keep
-        // their norm gets its numerators on FP64 MFMA; the others go to the
-        // device queue (fix_kernel recomputes them after the launch), or, when it
+        // flagged windows of the row group, after its tile loop: a tile of
+        // many windows that keep their norm is recorded for the tile launch
+        // (numerators on FP64 MFMA); the others go to the device queue
+        // (fix_kernel recomputes them after the launch), or, when it
         // is full, to the wave's list, recomputed here one window per lane
         // in passes of 64 (a few left at the end: the whole wave on one
         // window at a time).  List entry: tile (5 bits), step r (2 bits),
@@ -485,7 +535,7 @@ __global__ __launch_bounds__(NT, (td_blocks_per_cu<MT>())) void tdcorr_kernel(co
                     bool cr;
                     entryWindow(list[done + lane], wi, row, cr);
                     const double rho =
-                        exact_window_td(sm.raw, sm.P1, sm.P2, wi, to_global(row.tmpl), row.Lt, a, cr, 0, 1);
+                        exact_window_td(sm.raw, sm.P, wi, to_global(row.tmpl), row.Lt, a, cr, 0, 1);
                     to_global(static_cast<float *>(row.out))[base + wi] = static_cast<float>(rho);
                 }
                 done += n;
@@ -497,7 +547,7 @@ __global__ __launch_bounds__(NT, (td_blocks_per_cu<MT>())) void tdcorr_kernel(co
                     bool cr;
                     entryWindow(list[done], wi, row, cr);  // uniform entry: the wave shares it
                     const double rho =
-                        exact_window_td(sm.raw, sm.P1, sm.P2, wi, to_global(row.tmpl), row.Lt, a, cr, lane, 64);
+                        exact_window_td(sm.raw, sm.P, wi, to_global(row.tmpl), row.Lt, a, cr, lane, 64);
                     if (lane == 0) { to_global(static_cast<float *>(row.out))[base + wi] = static_cast<float>(rho); }
                 }
             } else if (done > 0) {
@@ -538,8 +588,8 @@ __global__ __launch_bounds__(NT, (td_blocks_per_cu<MT>())) void tdcorr_kernel(co
                 // row 4 r + quad of the result; its mark is bit quad of lane 16 r + c16
                 if ((fq[wave][tile][16 * r + c16] >> quad) & 1u) {
                     const TdRow row = rows[rowBase + 4 * r + quad];
-                    const double S1 = sm.P1[i + row.Lt] - sm.P1[i];
-                    const double den2 = row.Lt * (sm.P2[i + row.Lt] - sm.P2[i]) - S1 * S1;
+                    const double S1 = sm.P[i + row.Lt].s1 - sm.P[i].s1;
+                    const double den2 = row.Lt * (sm.P[i + row.Lt].s2 - sm.P[i].s2) - S1 * S1;
                     double rho = acc[r] * sqrt(row.Lt / den2);
                     if (fabs(rho) > 1.1) { rho = 0; }
                     to_global(static_cast<float *>(row.out))[base + i] = static_cast<float>(rho);
@@ -559,15 +609,6 @@ __global__ __launch_bounds__(NT, (td_blocks_per_cu<MT>())) void tdcorr_kernel(co
                 nCanc += static_cast<unsigned>(__popcll(__ballot(((flg & cnc) >> r) & 1u)));
             }
             unsigned keep = flg;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                if (((flg & cnc) >> r) & 1u) {
-                    if (constant_window(sm.eqw, i, LtR[r])) {
-                        outR[r][i] = 0.0f;
-                        keep &= ~(1u << r);
-                    }
-                }
-            }
             const unsigned noisy = keep & ~cnc;
             int n = 0, nNoisy = 0;
 #pragma unroll
@@ -576,9 +617,27 @@ __global__ __launch_bounds__(NT, (td_blocks_per_cu<MT>())) void tdcorr_kernel(co
                 nNoisy += __popcll(__ballot((noisy >> r) & 1u));
             }
             if (nNoisy >= kTdTileFlags) {
-                fq[wave][tile][lane] = static_cast<unsigned char>(noisy);
-                wave_lds_sync();
-                exactTile(tile);
+                // the tile launch's, marked by NaN; in place when its list is full
+                unsigned long long k = 0;
+                if (lane == 0) { k = atomicAdd(queue.overCount, 1ull); }
+                k = __shfl(k, 0, 64);
+                if (k < queue.overCap) {
+                    if (lane == 0) {
+                        gptr<int> rec = to_global(queue.over) + 4 * k;
+                        rec[0] = rowBase;
+                        rec[1] = nMine;
+                        rec[2] = static_cast<int>(base) + 16 * tile;
+                        rec[3] = 0;
+                    }
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        if ((noisy >> r) & 1u) { outR[r][i] = __builtin_nanf(""); }
+                    }
+                } else {
+                    fq[wave][tile][lane] = static_cast<unsigned char>(noisy);
+                    wave_lds_sync();
+                    exactTile(tile);
+                }
                 keep &= cnc;
                 n -= nNoisy;
             }
@@ -629,6 +688,105 @@ __global__ __launch_bounds__(NT, (td_blocks_per_cu<MT>())) void tdcorr_kernel(co
     }
 }
 
+// The recorded tiles of a time-domain launch, one wave each: the windows
+// marked NaN among 16 rows x 16 outputs are recomputed in FP64, numerators on
+// v_mfma_f64_16x16x4 and norms from prefix sums of the tile's own samples
+// (about the first of them).  A launch of its own because a gap's edge flags
+// every tile of a few items: recomputed inside them, those items ran three
+// to four times longer than the rest and the chip waited for them (0.8 of
+// 2.84 ms, 256 rows x 4 channels x 1 M samples).
+constexpr int kTileSpan = 320;  // samples a tile may read (16 + 255), five per lane
+__global__ __launch_bounds__(NT) void fix_tiles_kernel(const TdRow *__restrict__ rows, FixQueue queue)
+{
+    constexpr int PER = kTileSpan / 64;
+    __shared__ float rawS[NT / 64][kTileSpan];
+    __shared__ TdSums sumS[NT / 64][kTileSpan + 1];
+    const unsigned long long n = min(*queue.overCount, queue.overCap);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, quad = lane >> 4, c16 = lane & 15;
+    float *raw = rawS[wave];
+    TdSums *P = sumS[wave];
+    for (unsigned long long k = static_cast<unsigned long long>(blockIdx.x) * (NT / 64) + wave; k < n;
+         k += static_cast<unsigned long long>(gridDim.x) * (NT / 64)) {
+        const gptr<const int> rec = to_global(static_cast<const int *>(queue.over)) + 4 * k;
+        const int rowBase = __builtin_amdgcn_readfirstlane(rec[0]);
+        const int nMine = __builtin_amdgcn_readfirstlane(rec[1]);
+        const int pos = __builtin_amdgcn_readfirstlane(rec[2]);
+        const TdRow mine = rows[rowBase + min(c16, nMine - 1)];
+        const gptr<const double> t = to_global(mine.tmpl);
+        const int LtA = c16 < nMine ? mine.Lt : 0;
+        // the longest row, and the samples that some row's windows reach
+        int LtMax = mine.Lt, limit = static_cast<int>(mine.nOut) + mine.Lt - 1;
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) {
+            LtMax = max(LtMax, __shfl_xor(LtMax, o, 64));
+            limit = max(limit, __shfl_xor(limit, o, 64));
+        }
+        LtMax = __builtin_amdgcn_readfirstlane(LtMax);
+        const gptr<const float> x = to_global(mine.x);
+        const double a = static_cast<double>(x[pos]);
+        float v[PER];
+        double l1[PER], l2[PER], t1 = 0, t2 = 0;
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            const int j = lane * PER + q;
+            v[q] = pos + j < limit ? x[pos + j] : 0.0f;
+            const double d = pos + j < limit ? static_cast<double>(v[q]) - a : 0.0;
+            l1[q] = t1;
+            l2[q] = t2;
+            t1 += d;
+            t2 += d * d;
+        }
+        const double e1 = wave_scan_sum(t1) - t1, e2 = wave_scan_sum(t2) - t2;
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            raw[lane * PER + q] = v[q];
+            P[lane * PER + q] = TdSums{e1 + l1[q], e2 + l2[q]};
+        }
+        if (lane == 63) { P[kTileSpan] = TdSums{e1 + t1, e2 + t2}; }
+        wave_lds_sync();
+        f64x4 acc = {};
+        double tk[4];
+        const auto taps = [&](int k0) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int m = k0 + 4 * u + quad;
+                tk[u] = m < LtA ? t[m] : 0.0;
+            }
+        };
+        taps(0);
+        for (int k0 = 0; k0 < LtMax; k0 += 16) {
+            double tc[4], dk[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                tc[u] = tk[u];
+                dk[u] = static_cast<double>(raw[c16 + k0 + 4 * u + quad]) - a;
+            }
+            taps(k0 + 16);  // in flight through this step's products
+#pragma unroll
+            for (int u = 0; u < 4; ++u) { acc = __builtin_amdgcn_mfma_f64_16x16x4f64(tc[u], dk[u], acc, 0, 0, 0); }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int j = 4 * r + quad;  // the result's row
+            if (j < nMine) {
+                const TdRow row = rows[rowBase + j];
+                if (pos + c16 < row.nOut) {
+                    gptr<float> out = to_global(static_cast<float *>(row.out)) + pos + c16;
+                    if (isnan(*out)) {
+                        const double S1 = P[c16 + row.Lt].s1 - P[c16].s1;
+                        const double den2 = row.Lt * (P[c16 + row.Lt].s2 - P[c16].s2) - S1 * S1;
+                        double rho = acc[r] * sqrt(row.Lt / den2);
+                        if (fabs(rho) > 1.1) { rho = 0; }
+                        *out = static_cast<float>(rho);
+                    }
+                }
+            }
+        }
+        wave_lds_sync();  // the next record rewrites the wave's tables
+    }
+}
+
 // Split templates: frag[row] = the KT taps of each part in turn (hi, then
 // lo for FP16; hi, mid, lo for BF16), zero past Lt.  Each part rounds what
 // the parts before it left of the FP64 tap (the remainder is exact in FP64).
@@ -650,6 +808,13 @@ __global__ __launch_bounds__(NT) void td_prep_kernel(const TdPrepJob *__restrict
 }
 
 }  // namespace
+
+hipError_t launch_fix_tiles(const TdRow *dRows, FixQueue queue, int blocks, hipStream_t stream)
+{
+    if (blocks <= 0 || queue.over == nullptr) { return hipSuccess; }
+    hipLaunchKernelGGL(fix_tiles_kernel, dim3(blocks), dim3(NT), 0, stream, dRows, queue);
+    return hipGetLastError();
+}
 
 bool td_supported(int nb) { return nb >= 1 && nb <= kTdMaxTaps; }
 

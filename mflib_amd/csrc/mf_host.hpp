@@ -282,27 +282,38 @@ inline std::mutex &costMutex()
     return m;
 }
 
-// The FP32 default is mf_autotune's measurement on an MI355X (microseconds
-// per block for the whole GPU; variant 1 block-wide, 2 wave-level); FP64
-// starts from the static model below.
+// mf_autotune's measurements on an MI355X (microseconds per block for the
+// whole GPU; variant 1 block-wide, 2 wave-level).
 inline CostTable defaultCostTable(int precision)
 {
     CostTable t;
 #ifdef MF_STATIC_FORMULA
     return t;
 #endif
-    if (precision != MF_PRECISION_FLOAT) { return t; }
     struct E { int logM, v; double a, bS, bO; };
-    static const E kMi355x[] = {
-        {9, 1, 0.00949, 0.00331, 0.00551},  {9, 2, 0.01247, 0.00135, 0.00237},
-        {10, 1, 0.01468, 0.00583, 0.00882}, {10, 2, 0.02817, 0.00176, 0.00415},
-        {11, 1, 0.03286, 0.01595, 0.02210}, {11, 2, 0.05440, 0.00756, 0.00747},
-        {12, 1, 0.08531, 0.05636, 0.07194},
+    static const E kFloat[] = {
+        {9, 1, 0.01148, 0.00343, 0.00562},  {9, 2, 0.01264, 0.00094, 0.00191},
+        {10, 1, 0.01368, 0.00632, 0.00941}, {10, 2, 0.01912, 0.00202, 0.00400},
+        {11, 1, 0.03230, 0.01791, 0.02368}, {11, 2, 0.05032, 0.00670, 0.00660},
+        {12, 1, 0.07990, 0.06440, 0.08140},
     };
-    for (const E &e : kMi355x) {
+    // Without this table the static model put FP64 rows of 700 samples on
+    // blocks of 1024 (324 useful outputs): 24 channels x 0.9 M samples took
+    // 1.05 ms there and 0.64 ms on blocks of 2048.
+    static const E kDouble[] = {
+        {9, 1, 0.01082, 0.00502, 0.00865},  {9, 2, 0.01944, 0.00150, 0.00420},
+        {10, 1, 0.02061, 0.01210, 0.02054}, {10, 2, 0.03824, 0.00735, 0.00724},
+        {11, 1, 0.05057, 0.04029, 0.06305},
+    };
+    const auto put = [&t](const E &e) {
         t.a[e.logM][e.v] = e.a;
         t.bShared[e.logM][e.v] = e.bS;
         t.bSolo[e.logM][e.v] = e.bO;
+    };
+    if (precision == MF_PRECISION_FLOAT) {
+        for (const E &e : kFloat) { put(e); }
+    } else {
+        for (const E &e : kDouble) { put(e); }
     }
     t.measured = true;
     return t;

@@ -32,11 +32,12 @@
 // window's sum of (x - a)^2 and den its centred norm; eps_split is the
 // relative size of the dropped products and split residuals: 3 * 2^-22 for
 // the FP16 pair (3 u^2, u = 2^-11) and 3 * 2^-24 for the BF16 triple
-// (3 u^3, u = 2^-8).  Windows whose bound exceeds the FP32 tolerance get
-// their numerator recomputed in FP64 from the anchored samples (the window
-// norm from the prefix sums is accurate there); windows whose FP64
-// variance lost too many digits get the exact two-pass Pearson value, as
-// in the FFT path.
+// (3 u^3, u = 2^-8); the FP16 pair also loses low parts below its smallest
+// subnormal, at most 2^-25 of the block's RMS per sample.  Windows whose
+// bound exceeds the FP32 tolerance get their numerator recomputed in FP64
+// from the anchored samples (the window norm from the prefix sums is accurate
+// there); windows whose FP64 variance lost too many digits get the exact
+// two-pass Pearson value, as in the FFT path.
 #include "mf_device.hpp"
 #include "mf_kernels.hpp"
 #include <cfloat>
@@ -345,6 +346,7 @@ __global__ __launch_bounds__(NT, kTdBlocks) void tdcorr_kernel(const TdItem *__r
     const float scF = blk.scF;
     const float flK = blk.flK;
 
+    constexpr float kUnder = NP == 2 ? static_cast<float>(2.98023223876953125e-08 / kTdRhoTol) : 0.0f;
     unsigned long long nFlag = 0, nCanc = 0;  // windows recomputed by this wave, in full
     for (int g = 0; 64 * g < item.nRows; ++g) {
         const int rowBase = item.rowBegin + 64 * g + 16 * wave;
@@ -372,7 +374,7 @@ __global__ __launch_bounds__(NT, kTdBlocks) void tdcorr_kernel(const TdItem *__r
         // the epilogue constants of the lane's 4 rows (absent rows: no
         // outputs, and a length that keeps the prefix reads in the span)
         int LtR[4], nvR[4];
-        float kcR[4], knR[4], slR[4];
+        float kcR[4], knR[4], slR[4], floorF[4];
         gptr<float> outR[4];
         int fullOut = IS;  // outputs every row of the group has
 #pragma unroll
@@ -394,6 +396,11 @@ __global__ __launch_bounds__(NT, kTdBlocks) void tdcorr_kernel(const TdItem *__r
                 slR[r] = 0.0f;
                 outR[r] = nullptr;
             }
+            // below the cancellation floor, or (FP16) so quiet beside the
+            // block's RMS s that the samples' low parts underflow: their
+            // rounding, 2^-25 s each, is sqrt(Lt) 2^-25 s in the numerator
+            const float under = kUnder * scF * static_cast<float>(LtR[r]);
+            floorF[r] = fmaf(under, under, flK * static_cast<float>(LtR[r]));
             fullOut = min(fullOut, nvR[r]);
         }
         fullOut = min(fullOut, __shfl_xor(fullOut, 16, 64));
@@ -461,7 +468,7 @@ __global__ __launch_bounds__(NT, kTdBlocks) void tdcorr_kernel(const TdItem *__r
                         const TdSums pe = sm.P[i + LtR[r]];
                         const double S1 = pe.s1 - pi.s1, S2 = pe.s2 - pi.s2;
                         const float d2 = static_cast<float>(fma(-S1, S1, LtR[r] * S2));
-                        flags[r] = __ballot(!(fmaf(-knR[r], static_cast<float>(S2), d2) > flK * static_cast<float>(LtR[r])));
+                            flags[r] = __ballot(!(fmaf(-knR[r], static_cast<float>(S2), d2) > floorF[r]));
                         any |= flags[r];
                         float y = __builtin_amdgcn_rsqf(d2);
                         y = y * (1.5f - 0.5f * d2 * y * y);

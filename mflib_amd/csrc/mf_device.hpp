@@ -309,11 +309,6 @@ struct WavePlan<2048> {
 // Padded exchange index: one spare slot every 16 points breaks the
 // power-of-two strides of the Stockham stores across LDS banks.
 __device__ __forceinline__ int xpad(int i) { return i + (i >> 4); }
-template <int M>
-struct XBuf {
-    static constexpr int size = M + M / 16;
-};
-
 // Orders a wave's LDS stores before its later loads (LDS operations of one
 // wave complete in issue order; this stops the compiler from moving them).
 __device__ __forceinline__ void wave_lds_sync()
@@ -329,19 +324,6 @@ __device__ __forceinline__ void wave_lds_sync()
 // bits never carry), so each access is one base register plus an
 // immediate offset.
 constexpr int cpad(int i) { return i + (i >> 4); }
-
-template <typename T, int M, int R>
-__device__ __forceinline__ void wave_load(Cx<T> *v, const Cx<T> *buf, int lane)
-{
-    constexpr int B = M / (R * 64);
-    static_assert((M / R) % 16 == 0, "load offsets must be 16-aligned");
-    const Cx<T> *p = buf + xpad(lane);
-#pragma unroll
-    for (int b = 0; b < B; ++b) {
-#pragma unroll
-        for (int r = 0; r < R; ++r) { v[b * R + r] = p[cpad(64 * b + r * (M / R))]; }
-    }
-}
 
 // cos and sin of 2 pi num / den at compile time (Taylor series around 0
 // after reduction to an eighth of a turn).
@@ -486,40 +468,6 @@ __device__ __forceinline__ void wave_pass2(Cx<T> *v, const W &tw)
     }
 #pragma unroll
     for (int b = 0; b < B; ++b) { mfcl::dftR<R, true>(&v[b * R]); }
-}
-
-template <typename T, int M, int R, int NS>
-__device__ __forceinline__ void wave_store(const Cx<T> *v, Cx<T> *buf, int lane)
-{
-    constexpr int B = M / (R * 64);
-    static_assert(NS <= 64, "butterfly phase must depend on the lane only");
-    // j = lane + 64 b, k = j mod NS = lane mod NS:
-    // dst = (lane - k) R + k  +  64 b R + r NS
-    const int k = lane & (NS - 1);
-    Cx<T> *p = buf + xpad((lane - k) * R + k);
-#pragma unroll
-    for (int b = 0; b < B; ++b) {
-#pragma unroll
-        for (int r = 0; r < R; ++r) { p[cpad(64 * b * R + r * NS)] = v[b * R + r]; }
-    }
-}
-
-// Inverse passes 1 and 2 on data in registers (v[b R1 + r] = point lane +
-// 64 b + r M/R1), up to the inputs of pass 3.
-template <typename T, int M, typename W>
-__device__ __forceinline__ void wave_passes12(Cx<T> *v, Cx<T> *buf, int lane, const W &tw)
-{
-    using P = WavePlan<M>;
-    wave_pass1<T, M>(v);
-    wave_store<T, M, P::R1, 1>(v, buf, lane);
-    wave_lds_sync();
-    wave_load<T, M, P::R2>(v, buf, lane);
-    wave_pass2<T, M>(v, tw);
-    wave_lds_sync();
-    wave_store<T, M, P::R2, P::R1>(v, buf, lane);
-    wave_lds_sync();
-    wave_load<T, M, P::R3>(v, buf, lane);
-    wave_lds_sync();
 }
 
 // One radix-4 pass of a 256-point forward transform held as 4 points per
@@ -689,6 +637,7 @@ __device__ __forceinline__ void wave_exchange_split(Cx<T> *v, T *buf, int lane)
     for (int r = 0; r < RL; ++r) { v[r] = {x[r], q[72 * r]}; }
     wave_lds_sync();
 }
+// wave_passes12_half one component at a time.
 template <typename T, int M, typename W>
 __device__ __forceinline__ void wave_passes12_split(Cx<T> *v, T *buf, int lane, const W &tw)
 {
@@ -699,7 +648,8 @@ __device__ __forceinline__ void wave_passes12_split(Cx<T> *v, T *buf, int lane, 
     wave_exchange_split<T, M, P::R2, P::R1, P::R3>(v, buf, lane);
 }
 
-// wave_passes12 through a half buffer.
+// Inverse passes 1 and 2 on data in registers (v[b R1 + r] = point lane +
+// 64 b + r M/R1), up to the inputs of pass 3, through a half buffer.
 template <typename T, int M, typename W>
 __device__ __forceinline__ void wave_passes12_half(Cx<T> *v, Cx<T> *buf, int lane, const W &tw)
 {

@@ -594,8 +594,10 @@ __device__ __forceinline__ void fixup_row_wave(XPtr raw, const T *sc, gptr<const
 // Shape of corr2_kernel<T, M>:
 //  - SHARED: a block-wide scale buffer for groups of rows of one template
 //    length (FP32 up to M = 1024, FP64 up to M = 512);
-//  - HALF: half-size exchange buffers per wave (and a solo row's scale is
-//    computed half a block at a time);
+//  - PREFIX: solo scales (and the shared one) from an FP64 prefix table of
+//    every sample, exchanges one component at a time; the others keep tile
+//    sums, exchange through half-size buffers and compute a solo row's scale
+//    half a block at a time;
 //  - W2LDS, W3REG: where the pass-2 and pass-3 twiddles live (WaveTwiddles);
 //  - TILE: samples per FP64 prefix-sum tile (FP32: 4, or 8 at M = 2048; FP64:
 //    16, whose windows sum whole tiles);
@@ -621,7 +623,6 @@ template <typename T, int M>
 struct Corr2Shape {
     static constexpr bool F64 = sizeof(T) == 8;
     static constexpr bool SHARED = corr2_shared_scale(static_cast<int>(sizeof(T)), M);
-    static constexpr bool HALF = F64 || M >= 1024;
     static constexpr bool W2LDS = F64 || M == 1024;
     static constexpr bool W3REG = !F64 && M == 2048;
     static constexpr int TILE = F64 ? 16 : (M >= 2048 ? 8 : 4);
@@ -646,7 +647,6 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
     constexpr bool PREFIX = Shape::PREFIX;
     constexpr int TILE = Shape::TILE;
     constexpr bool SHARED = Shape::SHARED;
-    constexpr bool HALF = Shape::HALF;
     constexpr int NTILE = N / TILE;
     constexpr int SPT = N / NT;
     constexpr int LOGN = Log2<N>::value;
@@ -654,10 +654,10 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
     constexpr int NWAVE = NT / 64;
     constexpr int XH = XHalf<M>::size;
     // exchange buffer of one wave
-    constexpr int XW = PREFIX ? XSplit<M>::size / 2 : HALF ? XH : XBuf<M>::size;
+    constexpr int XW = PREFIX ? XSplit<M>::size / 2 : XH;
     using P = WavePlan<M>;
     static_assert(N % NT == 0, "block shape");
-    static_assert(2 * XH == XBuf<M>::size, "two half buffers make one full buffer");
+    static_assert(PREFIX || M <= XH * 2, "half a block's scales fit an exchange buffer");
     // PREFIX: the FP64 prefix sums at every sample, one spare entry per 16 so
     // that the 4 consecutive entries a thread writes spread over the LDS
     // banks, and GROUP - 1 entries past the end, which the reads for outputs
@@ -672,7 +672,7 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
     T *raw = PREFIX ? reinterpret_cast<T *>(pf) : rawBuf;
     __shared__ Cx<T> Xs[M];
     __shared__ __align__(16) T sc[SHARED ? N : 1];
-    // one exchange buffer per wave (half size with HALF)
+    // one exchange buffer per wave
     __shared__ Cx<T> xb[NWAVE * XW];
     using W = WaveTwiddles<T, M, Shape::W2LDS, Shape::W3REG>;
     __shared__ Cx<T> w2tab[W::TABLE];
@@ -864,10 +864,8 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
         }
         if constexpr (PREFIX) {
             wave_passes12_split<T, M>(v, reinterpret_cast<T *>(buf), lane, wt);
-        } else if constexpr (HALF) {
-            wave_passes12_half<T, M>(v, buf, lane, wt);
         } else {
-            wave_passes12<T, M>(v, buf, lane, wt);
+            wave_passes12_half<T, M>(v, buf, lane, wt);
         }
         wave_pass3_inverse<T, M>(v, wt);
     };
@@ -1097,18 +1095,6 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
                 if (anyFlag) { fixup_row_wave<T>(raw, own, tmplG, row.Lt, to_global(outRow), end, lane, a, first, sg.flagged); }
             }
         };
-        if constexpr (!HALF) {
-            // the whole row's scale at once (the full buffer holds N values)
-            int nf = 0;
-            if (nvRow > 0) { nf = ownScale(nvRow, 0); }
-            const bool anyFlag = __ballot(nf > 0) != 0ull;
-            wave_lds_sync();
-            epilogueHalf(Half0{}, own, 0, outRow, nvRow);
-            epilogueHalf(Half1{}, own, 0, outRow, nvRow);
-            flagged(nf, anyFlag, 0, nvRow);
-            wave_lds_sync();  // the next row reuses buf
-            return;
-        }
         // half 0: outputs [0, N/2)
         {
             const int n0 = min(nvRow, N / 2);

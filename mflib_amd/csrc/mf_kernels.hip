@@ -1232,7 +1232,7 @@ __global__ __launch_bounds__(NT) void tmpl_kernel(const TmplJob *__restrict__ jo
 
 // out[k] = sum_r w_r * |rho_r[k + s_r]| in row order, no contraction,
 // as the reference's shiftAndStack loop (src/matchedFilter.cpp:1341-1361).
-template <typename T>
+template <typename T, int U>
 __global__ __launch_bounds__(NT) void stack_kernel(const StackGroup *__restrict__ groups, int absval)
 {
     // hipcc contracts a*b+c into an FMA by default; the stack keeps the
@@ -1243,47 +1243,42 @@ __global__ __launch_bounds__(NT) void stack_kernel(const StackGroup *__restrict_
     const int nRows = grp.nRows;
     const long long len = grp.len;
     T *__restrict__ out = static_cast<T *>(grp.out);
-    // Each block owns one contiguous chunk of kStackChunk outputs, so the
-    // cache lines a block reads are shared only with the chunks beside it
-    // (neighbouring blocks sit on other XCDs, whose L2s would each fetch a
-    // shared line).  In a pass a thread owns U outputs NT apart, so every
-    // load instruction of a wave reads 64 consecutive samples of a row.
-    // The row loop is unrolled (8 rows: 64 loads in flight per thread;
-    // measured best against 4, 12, 16 and 24) so several rows' loads are in
-    // flight while the per-output sums keep their sequential order.
-    constexpr int U = 8;
-    static_assert(kStackChunk % (NT * U) == 0, "stack chunk");
-    const long long chunk0 = static_cast<long long>(blockIdx.x) * kStackChunk;
+    // Each block owns one contiguous chunk of NT U outputs, so the cache lines
+    // a block reads are shared only with the chunks beside it (neighbouring
+    // blocks sit on other XCDs, whose L2s would each fetch a shared line).  A
+    // thread owns U outputs NT apart, so every load instruction of a wave
+    // reads 64 consecutive samples of a row.  The row loop is unrolled (8
+    // rows: 64 loads in flight per thread at U = 8; measured best against 4,
+    // 12, 16 and 24) so several rows' loads are in flight while the
+    // per-output sums keep their sequential order.
+    const long long chunk0 = static_cast<long long>(blockIdx.x) * (NT * U);
     if (chunk0 >= len) { return; }
     gptr<T> o = to_global(out);
-    for (int pass = 0; pass < kStackChunk / (NT * U); ++pass) {
-        const long long k0 = chunk0 + static_cast<long long>(pass) * NT * U + threadIdx.x;
-        if (k0 >= len) { break; }
-        T acc[U];
+    const long long k0 = chunk0 + threadIdx.x;
+    T acc[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) { acc[u] = T(0); }
+    for (int u = 0; u < U; ++u) { acc[u] = T(0); }
 #pragma unroll 8
-        for (int r = 0; r < nRows; ++r) {
-            const StackRow sr = srows[r];
-            const gptr<const T> p = to_global(static_cast<const T *>(sr.rho)) + sr.shift;
-            const T w = static_cast<T>(sr.weight);
-            T v[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const long long k = k0 + u * NT;
-                v[u] = k < len ? p[k] : T(0);
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const T a = absval ? fabs(v[u]) : v[u];
-                acc[u] = acc[u] + w * a;
-            }
-        }
+    for (int r = 0; r < nRows; ++r) {
+        const StackRow sr = srows[r];
+        const gptr<const T> p = to_global(static_cast<const T *>(sr.rho)) + sr.shift;
+        const T w = static_cast<T>(sr.weight);
+        T v[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const long long k = k0 + u * NT;
-            if (k < len) { o[k] = acc[u]; }
+            v[u] = k < len ? p[k] : T(0);
         }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const T a = absval ? fabs(v[u]) : v[u];
+            acc[u] = acc[u] + w * a;
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const long long k = k0 + u * NT;
+        if (k < len) { o[k] = acc[u]; }
     }
 }
 
@@ -1490,24 +1485,22 @@ inline int peak_grid(long long maxLen, int tsize, int cap)
 }
 
 // Stack and candidates of every group in one launch (the detect path).  As
-// stack_kernel, each block owns kStackChunk outputs (one pass of U = 8 per
-// thread) and writes them; the block's sums also go to LDS, where each
+// stack_kernel, each block owns NT U outputs and writes them; the block's sums also go to LDS, where each
 // output above the threshold finds its neighbours.  An output at the
 // block's edge recomputes its outside neighbour from the rows: the same
 // sum, in the same order, as the block that owns it.  Candidates as in
 // peak_scan (the rule of src/peakFinder.cpp:500-521, one atomic per wave).
-template <typename T>
+template <typename T, int U>
 __global__ __launch_bounds__(NT) void stack_peak_kernel(const StackGroup *__restrict__ groups, int absval, T thr)
 {
 #pragma clang fp contract(off)
-    constexpr int U = 8;
-    static_assert(kStackChunk == NT * U, "one pass per block");
-    __shared__ T sv[kStackChunk];
+    constexpr int CH = NT * U;
+    __shared__ T sv[CH];
     const StackGroup grp = groups[blockIdx.y];
     const StackRow *__restrict__ srows = grp.rows;
     const int nRows = grp.nRows;
     const long long len = grp.len;
-    const long long chunk0 = static_cast<long long>(blockIdx.x) * kStackChunk;
+    const long long chunk0 = static_cast<long long>(blockIdx.x) * CH;
     if (chunk0 >= len) { return; }  // uniform per block
     const long long k0 = chunk0 + threadIdx.x;
     T acc[U];
@@ -1556,7 +1549,7 @@ __global__ __launch_bounds__(NT) void stack_peak_kernel(const StackGroup *__rest
         const T xi = acc[u];
         if (k < len && xi > thr) {
             const T left = j > 0 ? sv[j - 1] : (k > 0 ? stackAt(k - 1) : T(0));
-            const T right = k + 1 < len ? (j + 1 < kStackChunk ? sv[j + 1] : stackAt(k + 1)) : T(0);
+            const T right = k + 1 < len ? (j + 1 < CH ? sv[j + 1] : stackAt(k + 1)) : T(0);
             if (peak_rule(xi, left, right, k, len, thr)) { bits |= 1u << u; }
         }
     }
@@ -1735,11 +1728,21 @@ __global__ __launch_bounds__(NT) void seg_minmax_kernel(const Seg *__restrict__ 
     double lo = DBL_MAX, hi = -DBL_MAX;
     if (i0 < sg.n) {
         const gptr<const T> x = to_global(static_cast<const T *>(sg.x));
+        // Sixteen loads in flight per thread: a batch of few segments has few
+        // blocks, whose time is the latency of their loads in turn (24
+        // segments of 6511 samples: 8.9 -> 4.0 us).  A thread past the end
+        // reads the last sample again, which changes no minimum.
+        constexpr int U = 16;
         const long long i1 = min(sg.n, i0 + kDeadChunk);
-        for (long long i = i0 + threadIdx.x; i < i1; i += NT) {
-            const double v = static_cast<double>(x[i]);
-            lo = fmin(lo, v);
-            hi = fmax(hi, v);
+        for (long long i = i0 + threadIdx.x; i < i1; i += NT * U) {
+            T v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) { v[u] = x[min(i + u * NT, i1 - 1)]; }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                lo = fmin(lo, static_cast<double>(v[u]));
+                hi = fmax(hi, static_cast<double>(v[u]));
+            }
         }
     }
     const double bmax = block_max<NT>(hi, red);
@@ -2008,17 +2011,29 @@ hipError_t launch_tmpl(int precision, int logM, const TmplJob *dJobs, int nJobs,
     }
 }
 
+// Stacks of so few outputs that chunks of kStackChunk leave compute units idle
+// take chunks of kStackChunkFew: a block's time is its rows' load latency,
+// which more blocks share.  Stacks and candidates of 16 groups of 24 rows in
+// chunks of 2048 and of 512 outputs: 20,000 outputs (160 chunks of 2048) 16.8
+// and 14.0 us, 40,000 (320) 18.4 and 16.2, 60,000 (480) 20.2 and 22.8, 8.64 M
+// 2616 and 3311, so the line is at one and a half chunks per compute unit.
+static bool few_stack_chunks(long long chunks, int nGroups) { return chunks * nGroups < 384; }
+
 hipError_t launch_stack_groups(int precision, const StackGroup *dGroups, int nGroups, long long maxLen,
                                int absval, hipStream_t stream)
 {
     if (maxLen <= 0 || nGroups <= 0) { return hipSuccess; }
     const long long chunks = (maxLen + kStackChunk - 1) / kStackChunk;
     if (chunks > 0x7fffffffLL) { return hipErrorInvalidValue; }
-    const int grid = static_cast<int>(chunks);
+    const bool few = few_stack_chunks(chunks, nGroups);
+    const int outputs = few ? kStackChunkFew : kStackChunk;
+    const dim3 grid(static_cast<unsigned>((maxLen + outputs - 1) / outputs), static_cast<unsigned>(nGroups));
     if (precision == 0) {
-        hipLaunchKernelGGL(stack_kernel<float>, dim3(grid, nGroups), dim3(NT), 0, stream, dGroups, absval);
+        auto *k = few ? stack_kernel<float, kStackChunkFew / NT> : stack_kernel<float, kStackChunk / NT>;
+        hipLaunchKernelGGL(k, grid, dim3(NT), 0, stream, dGroups, absval);
     } else {
-        hipLaunchKernelGGL(stack_kernel<double>, dim3(grid, nGroups), dim3(NT), 0, stream, dGroups, absval);
+        auto *k = few ? stack_kernel<double, kStackChunkFew / NT> : stack_kernel<double, kStackChunk / NT>;
+        hipLaunchKernelGGL(k, grid, dim3(NT), 0, stream, dGroups, absval);
     }
     return hipGetLastError();
 }
@@ -2087,13 +2102,15 @@ hipError_t launch_stack_peak_groups(int precision, const StackGroup *dGroups, in
     if (maxLen <= 0 || nGroups <= 0) { return hipSuccess; }
     const long long chunks = (maxLen + kStackChunk - 1) / kStackChunk;
     if (chunks > 0x7fffffffLL || nGroups > 65535) { return hipErrorInvalidValue; }
-    const int grid = static_cast<int>(chunks);
+    const bool few = few_stack_chunks(chunks, nGroups);
+    const int outputs = few ? kStackChunkFew : kStackChunk;
+    const dim3 grid(static_cast<unsigned>((maxLen + outputs - 1) / outputs), static_cast<unsigned>(nGroups));
     if (precision == 0) {
-        hipLaunchKernelGGL(stack_peak_kernel<float>, dim3(grid, nGroups), dim3(NT), 0, stream, dGroups, absval,
-                           static_cast<float>(threshold));
+        auto *k = few ? stack_peak_kernel<float, kStackChunkFew / NT> : stack_peak_kernel<float, kStackChunk / NT>;
+        hipLaunchKernelGGL(k, grid, dim3(NT), 0, stream, dGroups, absval, static_cast<float>(threshold));
     } else {
-        hipLaunchKernelGGL(stack_peak_kernel<double>, dim3(grid, nGroups), dim3(NT), 0, stream, dGroups, absval,
-                           threshold);
+        auto *k = few ? stack_peak_kernel<double, kStackChunkFew / NT> : stack_peak_kernel<double, kStackChunk / NT>;
+        hipLaunchKernelGGL(k, grid, dim3(NT), 0, stream, dGroups, absval, threshold);
     }
     return hipGetLastError();
 }

@@ -9,7 +9,8 @@
 namespace mfk {
 
 constexpr int kThreads = 256;        // block size of every kernel here
-constexpr int kStackChunk = 2048;   // outputs per block of the stack kernel
+constexpr int kStackChunk = 2048;   // outputs per block of the stack kernels
+constexpr int kStackChunkFew = 512; // the same where there are few of them
 constexpr int kDeadChunk = 16384;   // samples per block of the segment dead-trace pass
 constexpr int kMinLogM = 9;          // smallest complex FFT size (M = 512)
 constexpr int kMaxLogMFloat = 12;    // M = 4096 (nfft 8192) in FP32

@@ -177,3 +177,27 @@ def test_lanczos_table_against_a_sine_per_tap(alpha):
         if np.sort(prof)[-2] < top - 1e-9:
             assert got[k] == pytest.approx(ref, abs=1e-12), (alpha, p)
     h.close()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("slen", [511, 512, 513, 1025, 383 * 2048, 383 * 2048 + 1])
+def test_stacks_on_either_side_of_the_chunk_rule(dtype, slen):
+    """Stacks cut into chunks of 512 outputs (383 chunks of 2048 and fewer) and
+    of 2048: both entry points equal the oracle's stack bit for bit, and every
+    local maximum is found, the chunk edges' included."""
+    rng = np.random.default_rng(slen)
+    C, L = 2, 40
+    shifts, weights = [0, 5], [0.625, 0.375]
+    n = L - 1 + slen + max(shifts)
+    h = capi.Handle(dtype, "batched")
+    h.set_templates([rng.standard_normal(L) for _ in range(C)], shifts=shifts, weights=weights)
+    h.set_batch_layout([n] * C, list(range(C)), [0] * C, 1)
+    h.initialize()
+    for c in range(C):
+        h.set_signal(c, rng.standard_normal(n).astype(dtype))
+    h.apply()
+    ref = O.shift_and_stack(np.stack([h.rho(r) for r in range(C)]), shifts, weights)
+    assert ref.size == slen
+    assert np.array_equal(h.detect(0.0, 0)[0], O.peak_finder(ref, 0.0, 0))
+    assert np.array_equal(h.shift_and_stack(0), ref)
+    h.close()

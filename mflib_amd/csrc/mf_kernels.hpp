@@ -65,7 +65,7 @@ struct FixQueue {
     // row blocks with flagged windows (row, first output, outputs), sized by
     // the host for every row block of the launches (two records per row block
     // at most), so they cannot overflow.  Time-domain kernel: tiles of many
-    // flagged windows (first row, rows, first output); past overCap a tile is
+    // flagged windows (first row, rows, first output, the item's anchor); past overCap a tile is
     // recomputed in place.
     unsigned long long *overCount;
     int *over;  // 4 ints per record
@@ -141,7 +141,7 @@ inline double td_eps(int kind, int KT)
 // One template row of a time-domain lane.  The epilogue's per-row
 // constants: with S1, S2 the window's sums of d = x - a and d^2 and
 // den2 = Lt S2 - S1^2, a window is recomputed in full when
-// den2 <= kc S2 + 1e-12 Lt E (E the block's sum of d^2: the variance lost
+// den2 <= kc S2 + 1e-9 Lt E (E the block's sum of d^2: the variance lost
 // its digits) and its numerator is recomputed when den2 < kn S2 (the
 // error bound exceeds the tolerance).
 struct TdRow {

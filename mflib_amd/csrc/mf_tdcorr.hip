@@ -88,6 +88,15 @@ constexpr int kTdCoopFlags = 4;  // at most this many left at the end: the wave 
 // 190 taps in 0.99 ms): the lines cross at 18.
 constexpr int kTdTileFlags = 20;
 
+// A window's norm is taken from the block's prefix sums when its den2 is above
+// kTdCancel Lt E (E the block's sum of d^2).  A prefix sum carries at most 14
+// roundings of values up to E (three samples of a thread, the wave's scan, the
+// waves before), so S2, a difference of two, is within 28 x 2^-53 E = 3.1e-15 E
+// and den2 within 3.1e-15 Lt E: 1.6e-6 of rho at this line.  Windows 90 dB below
+// their block take the two-pass value instead (|rho| 0.9 beside a spike of 1e7
+// times the noise was off by 1.6e-5 with a line of 1e-12).
+constexpr double kTdCancel = 1.0e-9;
+
 // FP64 prefix sums of d = x - a and of d^2 at one sample.
 struct __align__(16) TdSums {
     double s1, s2;
@@ -150,7 +159,7 @@ struct TdStage {
 };
 
 // What the epilogue needs of the staged block: the anchor a, the scale s
-// of x~ (FP32) and the cancellation floor 1e-12 E (per tap of Lt).
+// of x~ (FP32) and the cancellation floor kTdCancel E (per tap of Lt).
 struct TdBlock {
     double a;
     float scF;
@@ -272,7 +281,7 @@ __device__ __forceinline__ TdBlock td_stage(TdStage<MT, KT> &sm, const Seg &sg, 
         }
         __syncthreads();
     }
-    return TdBlock{a, static_cast<float>(sc), static_cast<float>(1.0e-12 * energy), any};
+    return TdBlock{a, static_cast<float>(sc), static_cast<float>(kTdCancel * energy), any};
 }
 
 // A dead lane's item: zeros in every row.
@@ -634,7 +643,7 @@ __global__ __launch_bounds__(NT, kTdBlocks) void tdcorr_kernel(const TdItem *__r
                         rec[0] = rowBase;
                         rec[1] = nMine;
                         rec[2] = static_cast<int>(base) + 16 * tile;
-                        rec[3] = 0;
+                        rec[3] = __float_as_int(static_cast<float>(a));  // a is an FP32 value
                     }
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
@@ -697,8 +706,11 @@ __global__ __launch_bounds__(NT, kTdBlocks) void tdcorr_kernel(const TdItem *__r
 
 // The recorded tiles of a time-domain launch, one wave each: the windows
 // marked NaN among 16 rows x 16 outputs are recomputed in FP64, numerators on
-// v_mfma_f64_16x16x4 and norms from prefix sums of the tile's own samples
-// (about the first of them).  A launch of its own because a gap's edge flags
+// v_mfma_f64_16x16x4 and norms from prefix sums of the tile's own samples,
+// about the anchor of the item that recorded them.  Their energy about it is
+// at most the item's, so the item's cancellation test holds for these sums
+// too; about a sample of the tile's own, which may be a spike or the end of a
+// loud stretch, it would not.  A launch of its own because a gap's edge flags
 // every tile of a few items: recomputed inside them, those items ran three
 // to four times longer than the rest and the chip waited for them (0.8 of
 // 2.84 ms, 256 rows x 4 channels x 1 M samples).
@@ -731,7 +743,7 @@ __global__ __launch_bounds__(NT) void fix_tiles_kernel(const TdRow *__restrict__
         }
         LtMax = __builtin_amdgcn_readfirstlane(LtMax);
         const gptr<const float> x = to_global(mine.x);
-        const double a = static_cast<double>(x[pos]);
+        const double a = static_cast<double>(__int_as_float(__builtin_amdgcn_readfirstlane(rec[3])));
         float v[PER];
         double l1[PER], l2[PER], t1 = 0, t2 = 0;
 #pragma unroll

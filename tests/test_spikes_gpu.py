@@ -1,0 +1,62 @@
+"""Isolated samples far above the signal's noise (a telemetry glitch, the last
+sample of a loud stretch) and runs of infinities: windows beside them keep the
+accuracy they have without them.  Correlations against the FP64 two-pass
+oracle."""
+import numpy as np
+import pytest
+
+import oracle as O
+from mflib_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+
+def _rows(tpls, x, dtype, nfft=0, variant=0):
+    h = capi.Handle(dtype, "batched")
+    h.set_templates(tpls)
+    h.set_batch_layout([x.size], [0] * len(tpls), [0] * len(tpls), 1)
+    if nfft:
+        h.set_fft_length(nfft)
+    if variant:
+        h.set_kernel_variant(variant)
+    h.initialize()
+    h.set_signal(0, x)
+    h.apply()
+    out = [h.rho(r) for r in range(len(tpls))]
+    stats = h.window_stats()
+    h.close()
+    return out, stats
+
+
+def _templates(rng, lengths):
+    return [rng.standard_normal(L) * np.hanning(L) for L in lengths]
+
+
+def _spiked(rng, tpls, at, amp, n):
+    """Unit noise, a spike of `amp` at every position of `at`, and right after
+    each a copy of one template four times the noise (|rho| about 0.9, where an
+    error of the window's norm shows in full)."""
+    x = rng.standard_normal(n)
+    for k, p in enumerate(at):
+        t = tpls[k % len(tpls)]
+        x[p + 1 + k % 5:][:t.size] += 4.0 * t
+    x[at] = amp * np.where(np.arange(len(at)) % 2, -0.9, 1.0)
+    return x
+
+
+@pytest.mark.parametrize("amp", [3.0e4, 3.0e5, 1.0e6, 1.0e7])
+@pytest.mark.parametrize("variant", [3, 4])
+@pytest.mark.parametrize("lengths", [(200,) * 24, tuple(range(230, 257)), (60,) * 20])
+def test_time_domain_windows_beside_a_spike(variant, lengths, amp):
+    """Spikes at every position within a tile of 16 outputs: the windows after
+    one are quiet beside their block and are recomputed, whole tiles of them."""
+    rng = np.random.default_rng(61)
+    tpls = _templates(rng, lengths)
+    n = 40_000
+    at = 1_000 + 1_201 * np.arange(32)  # 1201 = 1 modulo 16
+    x = _spiked(rng, tpls, at, amp, n).astype(np.float32)
+    out, _ = _rows(tpls, x, np.float32, variant=variant)
+    for r, t in enumerate(tpls):
+        ref = O.pearson(t, x)[:out[r].size]
+        err = np.abs(out[r].astype(np.float64) - ref)
+        assert err.max() < 1e-5, (r, int(err.argmax()), err.max())

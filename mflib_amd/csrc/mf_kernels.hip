@@ -712,13 +712,17 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
 
     // A. load, anchor, tile sums, energy.  Each thread takes SPT consecutive
     // samples, so tile sums and their scan stay in registers and DPP moves.
-    // The anchor a removes the block's offset: any value near the samples
-    // will do (the templates have zero mean, and the error model takes the
-    // energy about a), so every wave takes the same mean of 64 samples
-    // spread over the block, and no barrier is needed before the sums.
+    // The anchor a removes the block's offset.  In FP32 any value near the
+    // samples will do (the templates have zero mean, and the error model takes
+    // the energy about a), so every wave takes the same mean of 64 samples
+    // spread over the block, and no barrier is needed before the sums.  In
+    // FP64 the window sums' digits are the result's: the anchor is the block's
+    // mean, which a spike of size A moves by A / N (by A / 64, a spike of 1e4
+    // times the noise cost 1e-11 of rho over its block).
     const gptr<const T> x = to_global(static_cast<const T *>(sg.x)) + base;
     const int nSamp = static_cast<int>(min(static_cast<long long>(N), sg.n - base));
-    const T spread = x[min(lane * (N / 64), nSamp - 1)];
+    T spread = T(0);
+    if constexpr (!Shape::F64) { spread = x[min(lane * (N / 64), nSamp - 1)]; }
     T v0[SPT];
     const int j0 = tid * SPT;
     if (nSamp == N) {
@@ -734,7 +738,21 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
 #pragma unroll
         for (int q = 0; q < SPT; ++q) { v0[q] = j0 + q < nSamp ? x[j0 + q] : T(0); }
     }
-    const T aT = read_lane(wave_scan_sum(spread * T(1.0 / 64)), 63);
+    T aT;
+    if constexpr (Shape::F64) {
+        T s = T(0);
+#pragma unroll
+        for (int q = 0; q < SPT; ++q) { s += v0[q]; }
+        s = wave_scan_sum(s);
+        if (lane == 63) { red[wave] = s; }
+        __syncthreads();
+        s = red[0];
+#pragma unroll
+        for (int w = 1; w < NWAVE; ++w) { s += red[w]; }
+        aT = uniform(s / nSamp);
+    } else {
+        aT = read_lane(wave_scan_sum(spread * T(1.0 / 64)), 63);
+    }
     const double a = static_cast<double>(aT);
     constexpr int STEP = PREFIX ? 1 : TILE;         // samples between the sums kept
     double l1[SPT / STEP + 1], l2[SPT / STEP + 1];  // running sums there, then the thread's totals

@@ -60,3 +60,30 @@ def test_time_domain_windows_beside_a_spike(variant, lengths, amp):
         ref = O.pearson(t, x)[:out[r].size]
         err = np.abs(out[r].astype(np.float64) - ref)
         assert err.max() < 1e-5, (r, int(err.argmax()), err.max())
+
+
+@pytest.mark.parametrize("nfft", [1024, 2048])
+@pytest.mark.parametrize("lengths", [(300,), (300,) * 5, (300, 250, 120)])
+def test_fp64_windows_far_from_a_spike(nfft, lengths):
+    """Spikes at multiples of 1/64 of a block and as the last sample of a short
+    last block.  The anchor moves by amp / nfft, and window sums about it lose
+    (amp / nfft)^2 2^-53 of the noise's: under 1e-12 with the other roundings.
+    The windows that a spike has left fewer than 24 outputs before are not
+    compared here (a sliding sum keeps 2^-53 amp^2 of it over a run of outputs)."""
+    rng = np.random.default_rng(67)
+    tpls = _templates(rng, lengths)
+    nb = max(lengths)
+    step = (nfft - nb + 1) & ~1
+    for amp in (1.0e4, 3.0e4):
+        n = 4 * step + nfft // 8 + nb
+        at = np.array([0, nfft // 2, step + 5 * nfft // 64, 3 * step + 40 * nfft // 64, n - 1])
+        x = rng.standard_normal(n)
+        x[at] = amp
+        out, _ = _rows(tpls, x, np.float64, nfft=nfft, variant=2)
+        far = np.ones(out[0].size, dtype=bool)
+        for p in at:
+            far[p + 1:p + 25] = False
+        for r, t in enumerate(tpls):
+            ref = O.pearson(t, x)[:out[r].size]
+            err = np.abs(out[r] - ref)[far]
+            assert err.max() < 1e-12, (amp, r, err.max())

@@ -1066,7 +1066,8 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
                 const bool canc = fl && !(den2 > rs.kc);
                 nFlag += __popcll(__ballot(fl));
                 nCanc += __popcll(__ballot(canc));
-                const bool flat = canc && constant_window(eqw, i, row.Lt);
+                // (equal infinities have no mean: NaN, like every window that touches one)
+                const bool flat = canc && energyU < INFINITY && constant_window(eqw, i, row.Lt);
                 if (flat) { outG[i] = T(0); }
                 const unsigned long long m = __ballot(fl && !flat);
                 if (m == 0ull) { continue; }

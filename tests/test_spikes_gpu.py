@@ -87,3 +87,31 @@ def test_fp64_windows_far_from_a_spike(nfft, lengths):
             ref = O.pearson(t, x)[:out[r].size]
             err = np.abs(out[r] - ref)[far]
             assert err.max() < 1e-12, (amp, r, err.max())
+
+
+@pytest.mark.parametrize("rows", [1, 5])
+def test_server_runs_of_infinities(rows):
+    """A run of equal infinities has no finite mean, so its windows are NaN, as
+    are all that touch it, for rows that share a scale and for a row alone; a
+    run of equal finite samples stays 0 and the other windows exact."""
+    rng = np.random.default_rng(71)
+    tpls = _templates(rng, (100,) * rows)
+    n = 3_000
+    x = rng.standard_normal(n).astype(np.float32)
+    x[700:1_000] = np.inf
+    x[1_600:1_900] = np.float32(2.5)
+    srv = capi.Server(np.float32, budget_bytes=1 << 28, max_batch=4, max_inflight=1)
+    ids = srv.add_templates(tpls)
+    rid = srv.submit([x], ids)
+    srv.wait(rid)
+    clean = np.where(np.isinf(x), np.float32(0), x)
+    for r, t in enumerate(tpls):
+        row = srv.rho(rid, r, 0)
+        i = np.arange(row.size)
+        touched = (i + 99 >= 700) & (i < 1_000)
+        assert np.isnan(row[touched]).all(), np.flatnonzero(~np.isnan(row) & touched)
+        assert not row[1_600:1_801].any()
+        ref = O.pearson(t, clean)[:row.size]
+        assert np.abs(row[~touched] - ref[~touched]).max() < 1e-5
+    srv.release(rid)
+    srv.close()

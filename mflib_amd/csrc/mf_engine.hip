@@ -596,15 +596,18 @@ void initialize(mf_handle *h)
     if (!tdRows.empty()) {
         // room for 1 in 32 windows flagged (more are recomputed in place)
         const long long cap = std::min<long long>(std::max<long long>(tdWindows / 32, 1 << 16), 1 << 25);
-        // and for one in 16 tiles of 256 windows recorded
-        const long long tiles = std::min<long long>(std::max<long long>(tdWindows / (16 * 256), 1 << 12), 1 << 22);
+        // and for every tile of 16 outputs and up to 16 rows recorded (a group
+        // of one row records none): 16 bytes beside 64 bytes of results a row
+        long long tiles = 0;
+        for (const mfk::TdItem &it : tdItems) {
+            tiles += static_cast<long long>((it.nRows + 14) / 16) * (mfk::kTdOutputsPerItem / 16);
+        }
         h->dTdFix.alloc(256 + static_cast<size_t>(cap) * 8 + static_cast<size_t>(tiles) * 16);
         h->tdFix.count = h->dTdFix.as<unsigned long long>();
         h->tdFix.overCount = h->tdFix.count + 1;  // cleared together
         h->tdFix.entries = reinterpret_cast<int *>(static_cast<char *>(h->dTdFix.p) + 256);
         h->tdFix.cap = static_cast<unsigned long long>(cap);
         h->tdFix.over = h->tdFix.entries + 2 * cap;
-        h->tdFix.overCap = static_cast<unsigned long long>(tiles);
     }
     h->dTdItems.alloc(std::max<size_t>(tdItems.size(), 1) * sizeof(mfk::TdItem));
     if (!tdRows.empty()) {
@@ -661,7 +664,6 @@ void initialize(mf_handle *h)
             h->dFftFix.alloc(256 + static_cast<size_t>(2 * rowBlocks) * 16);
             h->fftFix.overCount = h->dFftFix.as<unsigned long long>();
             h->fftFix.over = reinterpret_cast<int *>(static_cast<char *>(h->dFftFix.p) + 256);
-            h->fftFix.overCap = static_cast<unsigned long long>(2 * rowBlocks);
         }
     }
     for (const auto &kv : tdLaunch) {

@@ -61,15 +61,13 @@ struct FixQueue {
     unsigned long long *count;
     int *entries;  // 8 bytes per entry
     unsigned long long cap;
-    // Records for a launch of their own, overCap of them.  FFT wave kernel:
-    // row blocks with flagged windows (row, first output, outputs), sized by
-    // the host for every row block of the launches (two records per row block
-    // at most), so they cannot overflow.  Time-domain kernel: tiles of many
-    // flagged windows (first row, rows, first output, the item's anchor); past overCap a tile is
-    // recomputed in place.
+    // Records for a launch of their own, room for every one that the launches
+    // can make, so they cannot overflow.  FFT wave kernel: row blocks with
+    // flagged windows (row, first output, outputs), two records per row block
+    // at most.  Time-domain kernel: tiles of many flagged windows (first row,
+    // rows, first output, the item's anchor).
     unsigned long long *overCount;
     int *over;  // 4 ints per record
-    unsigned long long overCap;
 };
 
 // One work item: block `block` of lane `seg`, for the first nRows rows of

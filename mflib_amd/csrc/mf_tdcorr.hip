@@ -87,6 +87,7 @@ constexpr int kTdCoopFlags = 4;  // at most this many left at the end: the wave 
 // the queue kernel (227 SIMD cycles each, measured: 10.7 M windows of about
 // 190 taps in 0.99 ms): the lines cross at 18.
 constexpr int kTdTileFlags = 20;
+static_assert(kTdTileFlags > 16, "the host counts no tiles of a group of one row");
 
 // A window's norm is taken from the block's prefix sums when its den2 is above
 // kTdCancel Lt E (E the block's sum of d^2).  A prefix sum carries at most 14
@@ -575,43 +576,6 @@ __global__ __launch_bounds__(NT, kTdBlocks) void tdcorr_kernel(const TdItem *__r
             }
             nList -= done;
         };
-        // The windows of a tile marked in the low bits of fq: numerators
-        // sum t (x - a) of all 16 x 16 by v_mfma_f64_16x16x4 (row lane % 16
-        // of the taps, column lane % 16 of the Hankel operand, k = lane / 16;
-        // result row 4 r + lane / 16), norms from the FP64 prefix sums.
-        auto exactTile = [&](int tile) {
-            const int i = 16 * tile + c16;
-            const TdRow mine = rows[rowBase + min(c16, nMine - 1)];
-            const gptr<const double> t = to_global(mine.tmpl);
-            const int LtA = c16 < nMine ? mine.Lt : 0;
-            int LtMax = max(max(LtR[0], LtR[1]), max(LtR[2], LtR[3]));
-            LtMax = max(LtMax, __shfl_xor(LtMax, 16, 64));
-            LtMax = __builtin_amdgcn_readfirstlane(max(LtMax, __shfl_xor(LtMax, 32, 64)));
-            f64x4 acc = {};
-            for (int k0 = 0; k0 < LtMax; k0 += 16) {  // LtMax <= KT, a multiple of 16
-                double tk[4], dk[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const int k = k0 + 4 * u + quad;
-                    tk[u] = k < LtA ? t[k] : 0.0;
-                    dk[u] = static_cast<double>(sm.raw[i + k]) - a;
-                }
-#pragma unroll
-                for (int u = 0; u < 4; ++u) { acc = __builtin_amdgcn_mfma_f64_16x16x4f64(tk[u], dk[u], acc, 0, 0, 0); }
-            }
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                // row 4 r + quad of the result; its mark is bit quad of lane 16 r + c16
-                if ((fq[wave][tile][16 * r + c16] >> quad) & 1u) {
-                    const TdRow row = rows[rowBase + 4 * r + quad];
-                    const double S1 = sm.P[i + row.Lt].s1 - sm.P[i].s1;
-                    const double den2 = row.Lt * (sm.P[i + row.Lt].s2 - sm.P[i].s2) - S1 * S1;
-                    double rho = acc[r] * sqrt(row.Lt / den2);
-                    if (fabs(rho) > 1.1) { rho = 0; }
-                    to_global(static_cast<float *>(row.out))[base + i] = static_cast<float>(rho);
-                }
-            }
-        };
         while (tiles != 0u) {
             const int tile = __ffs(tiles) - 1;
             tiles &= tiles - 1u;
@@ -619,40 +583,28 @@ __global__ __launch_bounds__(NT, kTdBlocks) void tdcorr_kernel(const TdItem *__r
             const unsigned word = fq[wave][tile][lane];
             const unsigned flg = word & 15u;
             const unsigned cnc = word >> 4;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                nFlag += static_cast<unsigned>(__popcll(__ballot((flg >> r) & 1u)));
-                nCanc += static_cast<unsigned>(__popcll(__ballot(((flg & cnc) >> r) & 1u)));
-            }
-            unsigned keep = flg;
-            const unsigned noisy = keep & ~cnc;
+            unsigned keep = flg;  // the window queue's
+            const unsigned noisy = flg & ~cnc;
             int n = 0, nNoisy = 0;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                n += __popcll(__ballot((keep >> r) & 1u));
+                n += __popcll(__ballot((flg >> r) & 1u));
                 nNoisy += __popcll(__ballot((noisy >> r) & 1u));
             }
-            if (nNoisy >= kTdTileFlags) {
-                // the tile launch's, marked by NaN; in place when its list is full
-                unsigned long long k = 0;
-                if (lane == 0) { k = atomicAdd(queue.overCount, 1ull); }
-                k = __shfl(k, 0, 64);
-                if (k < queue.overCap) {
-                    if (lane == 0) {
-                        gptr<int> rec = to_global(queue.over) + 4 * k;
-                        rec[0] = rowBase;
-                        rec[1] = nMine;
-                        rec[2] = static_cast<int>(base) + 16 * tile;
-                        rec[3] = __float_as_int(static_cast<float>(a));  // a is an FP32 value
-                    }
+            nFlag += static_cast<unsigned>(n);
+            nCanc += static_cast<unsigned>(n - nNoisy);
+            if (nNoisy >= kTdTileFlags) {  // the tile launch's, marked by NaN
+                if (lane == 0) {
+                    // the list has a record for every tile of the launch
+                    gptr<int> rec = to_global(queue.over) + 4 * atomicAdd(queue.overCount, 1ull);
+                    rec[0] = rowBase;
+                    rec[1] = nMine;
+                    rec[2] = static_cast<int>(base) + 16 * tile;
+                    rec[3] = __float_as_int(static_cast<float>(a));  // a is an FP32 value
+                }
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        if ((noisy >> r) & 1u) { outR[r][i] = __builtin_nanf(""); }
-                    }
-                } else {
-                    fq[wave][tile][lane] = static_cast<unsigned char>(noisy);
-                    wave_lds_sync();
-                    exactTile(tile);
+                for (int r = 0; r < 4; ++r) {
+                    if ((noisy >> r) & 1u) { outR[r][i] = __builtin_nanf(""); }
                 }
                 keep &= cnc;
                 n -= nNoisy;
@@ -720,7 +672,7 @@ __global__ __launch_bounds__(NT) void fix_tiles_kernel(const TdRow *__restrict__
     constexpr int PER = kTileSpan / 64;
     __shared__ float rawS[NT / 64][kTileSpan];
     __shared__ TdSums sumS[NT / 64][kTileSpan + 1];
-    const unsigned long long n = min(*queue.overCount, queue.overCap);
+    const unsigned long long n = *queue.overCount;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63, quad = lane >> 4, c16 = lane & 15;
     float *raw = rawS[wave];

@@ -115,3 +115,32 @@ def test_server_runs_of_infinities(rows):
         assert np.abs(row[~touched] - ref[~touched]).max() < 1e-5
     srv.release(rid)
     srv.close()
+
+
+@pytest.mark.parametrize("variant", [3, 4])
+@pytest.mark.parametrize("rows", [2, 17, 18, 40])
+def test_time_domain_most_tiles_noisy(variant, rows):
+    """A level that steps by 60 times the noise every 400 samples puts the noise
+    bound of the windows between steps above the tolerance, so most tiles of two
+    rows or more are recorded for recomputation, the same way in every pass."""
+    rng = np.random.default_rng(73)
+    tpls = _templates(rng, rng.integers(100, 129, size=rows))
+    n = 6_000
+    x = (rng.standard_normal(n) + 60.0 * (np.arange(n) // 400 % 2) + 500.0).astype(np.float32)
+    h = capi.Handle(np.float32, "batched")
+    h.set_templates(tpls)
+    h.set_batch_layout([n], [0] * rows, [0] * rows, 1)
+    h.set_kernel_variant(variant)
+    h.initialize()
+    h.set_signal(0, x)
+    h.apply()
+    out = [h.rho(r) for r in range(rows)]
+    ws = h.window_stats()
+    assert ws["flagged"] > 0.5 * ws["windows"] and ws["full"] == 0, ws
+    for r, t in enumerate(tpls):
+        ref = O.pearson(t, x)[:out[r].size]
+        assert np.abs(out[r].astype(np.float64) - ref).max() < 1e-5, r
+    h.apply()
+    for r in range(rows):
+        assert np.array_equal(h.rho(r), out[r]), r
+    h.close()

@@ -686,23 +686,24 @@ __global__ __launch_bounds__(NT) void fix_tiles_kernel(const TdRow *__restrict__
         const TdRow mine = rows[rowBase + min(c16, nMine - 1)];
         const gptr<const double> t = to_global(mine.tmpl);
         const int LtA = c16 < nMine ? mine.Lt : 0;
-        // the longest row, and the samples that some row's windows reach
-        int LtMax = mine.Lt, limit = static_cast<int>(mine.nOut) + mine.Lt - 1;
+        // the longest row, and the samples from pos on that the windows reach:
+        // no others, whose value (a NaN, a spike) the item's test has not seen
+        int LtMax = mine.Lt, reach = static_cast<int>(min(mine.nOut - pos, 16ll)) + mine.Lt - 1;
 #pragma unroll
         for (int o = 1; o < 16; o <<= 1) {
             LtMax = max(LtMax, __shfl_xor(LtMax, o, 64));
-            limit = max(limit, __shfl_xor(limit, o, 64));
+            reach = max(reach, __shfl_xor(reach, o, 64));
         }
         LtMax = __builtin_amdgcn_readfirstlane(LtMax);
-        const gptr<const float> x = to_global(mine.x);
+        const gptr<const float> x = to_global(mine.x) + pos;
         const double a = static_cast<double>(__int_as_float(__builtin_amdgcn_readfirstlane(rec[3])));
         float v[PER];
         double l1[PER], l2[PER], t1 = 0, t2 = 0;
 #pragma unroll
         for (int q = 0; q < PER; ++q) {
             const int j = lane * PER + q;
-            v[q] = pos + j < limit ? x[pos + j] : 0.0f;
-            const double d = pos + j < limit ? static_cast<double>(v[q]) - a : 0.0;
+            v[q] = j < reach ? x[j] : 0.0f;
+            const double d = j < reach ? static_cast<double>(v[q]) - a : 0.0;
             l1[q] = t1;
             l2[q] = t2;
             t1 += d;
@@ -742,7 +743,7 @@ __global__ __launch_bounds__(NT) void fix_tiles_kernel(const TdRow *__restrict__
             const int j = 4 * r + quad;  // the result's row
             if (j < nMine) {
                 const TdRow row = rows[rowBase + j];
-                if (pos + c16 < row.nOut) {
+                if (static_cast<long long>(pos) + c16 < row.nOut) {
                     gptr<float> out = to_global(static_cast<float *>(row.out)) + pos + c16;
                     if (isnan(*out)) {
                         const double S1 = P[c16 + row.Lt].s1 - P[c16].s1;

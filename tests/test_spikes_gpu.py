@@ -144,3 +144,28 @@ def test_time_domain_most_tiles_noisy(variant, rows):
     for r in range(rows):
         assert np.array_equal(h.rho(r), out[r]), r
     h.close()
+
+
+@pytest.mark.parametrize("variant", [3, 4])
+@pytest.mark.parametrize("lt", [128, 256])
+@pytest.mark.parametrize("bad", [np.nan, np.inf, 1.0e9])
+def test_sample_just_past_a_tile(variant, lt, bad):
+    """The recorded tiles at the end of an item of 512 outputs, whose windows end
+    just before a bad sample that the item does not read."""
+    rng = np.random.default_rng(79)
+    tpls = _templates(rng, (lt,) * 16)
+    n, end = 3_000, 512 + lt  # the item's samples are [0, 512 + lt)
+    x = (rng.standard_normal(n) + 60.0 * (np.arange(n) >= 400)).astype(np.float32)
+    x[end:end + 3] = bad
+    out, _ = _rows(tpls, x, np.float32, variant=variant)
+    i = np.arange(out[0].size)
+    touched = (i + lt > end) & (i < end + 3)
+    assert not touched[:512].any() and touched[513]
+    if np.isfinite(bad):
+        touched[:] = False
+    clean = np.where(np.isfinite(x), x, np.float32(0))
+    for r, t in enumerate(tpls):
+        assert not np.isnan(bad) or np.isnan(out[r][touched]).all()
+        ref = O.pearson(t, clean)[:out[r].size]
+        err = np.abs(out[r].astype(np.float64) - ref)[~touched]
+        assert err.max() < 1e-5, (r, np.flatnonzero(~touched)[err.argmax()], err.max())

@@ -2128,7 +2128,7 @@ int mf_set_signal_device(mf_handle *h, int channel, int n, const void *dx)
             MF_HIP(hipMemcpyAsync(c.buf.p, dx, static_cast<size_t>(n) * h->tsize, hipMemcpyDefault, h->stream));
             src = c.buf.p;
         }
-        const int nb = static_cast<int>(std::min<long long>((n + 2047) / 2048, 1024));
+        const int nb = static_cast<int>(std::min<long long>((n + 2047ll) / 2048, 1024));
         h->hMinMax.reserve(static_cast<size_t>(nb) * 2 * sizeof(double));
         const double *part = static_cast<const double *>(h->hMinMax.p);
         MF_HIP(mfk::launch_copy_minmax(h->precision, src, c.buf.p, n, static_cast<double *>(h->hMinMax.p), nb, h->stream));

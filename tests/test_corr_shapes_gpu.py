@@ -201,3 +201,21 @@ def test_stacks_on_either_side_of_the_chunk_rule(dtype, slen):
     assert np.array_equal(h.detect(0.0, 0)[0], O.peak_finder(ref, 0.0, 0))
     assert np.array_equal(h.shift_and_stack(0), ref)
     h.close()
+
+
+def test_device_signal_of_almost_2_31_samples():
+    """A signal handed over in device memory, so long that its length plus a
+    block's share leaves the range of int."""
+    torch = pytest.importorskip("torch")
+    n = 2 ** 31 - 1_000
+    x = torch.zeros(n, dtype=torch.float32, device="cuda")
+    x[-3:] = torch.tensor([1.0, -2.0, 0.5], device="cuda")
+    torch.cuda.synchronize()
+    h = capi.Handle(np.float32, "single")
+    h.set_templates([np.hanning(60)])
+    h.set_signal_size(n)
+    h.initialize()
+    h.set_signal_device(0, x.data_ptr(), n)
+    got = h.get_signal(0, n)[-4:]
+    assert np.array_equal(got, np.array([0.0, 1.0, -2.0, 0.5], dtype=np.float32))
+    h.close()

@@ -411,6 +411,10 @@ __global__ __launch_bounds__(NT, kTdBlocks) void tdcorr_kernel(const TdItem *__r
             // rounding, 2^-25 s each, is sqrt(Lt) 2^-25 s in the numerator
             const float under = kUnder * scF * static_cast<float>(LtR[r]);
             floorF[r] = fmaf(under, under, flK * static_cast<float>(LtR[r]));
+            // An absent row flags nothing: its one-sample windows have no norm,
+            // and with the block's floor every tile of a group of fewer than 16
+            // rows took the branch for flagged windows.
+            if (j >= nMine) { floorF[r] = -INFINITY; }
             fullOut = min(fullOut, nvR[r]);
         }
         fullOut = min(fullOut, __shfl_xor(fullOut, 16, 64));
@@ -478,7 +482,7 @@ __global__ __launch_bounds__(NT, kTdBlocks) void tdcorr_kernel(const TdItem *__r
                         const TdSums pe = sm.P[i + LtR[r]];
                         const double S1 = pe.s1 - pi.s1, S2 = pe.s2 - pi.s2;
                         const float d2 = static_cast<float>(fma(-S1, S1, LtR[r] * S2));
-                            flags[r] = __ballot(!(fmaf(-knR[r], static_cast<float>(S2), d2) > floorF[r]));
+                        flags[r] = __ballot(!(fmaf(-knR[r], static_cast<float>(S2), d2) > floorF[r]));
                         any |= flags[r];
                         float y = __builtin_amdgcn_rsqf(d2);
                         y = y * (1.5f - 0.5f * d2 * y * y);

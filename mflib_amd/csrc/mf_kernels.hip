@@ -722,7 +722,7 @@ __global__ __launch_bounds__(NT, (Corr2Shape<T, M>::BLOCKS)) void corr2_kernel(c
     const gptr<const T> x = to_global(static_cast<const T *>(sg.x)) + base;
     const int nSamp = static_cast<int>(min(static_cast<long long>(N), sg.n - base));
     T spread = T(0);
-    if constexpr (!Shape::F64) { spread = x[min(lane * (N / 64), nSamp - 1)]; }
+    if constexpr (!Shape::F64) { spread = x[(lane * nSamp) >> 6]; }
     T v0[SPT];
     const int j0 = tid * SPT;
     if (nSamp == N) {

@@ -188,7 +188,7 @@ __device__ __forceinline__ TdBlock td_stage(TdStage<MT, KT> &sm, const Seg &sg, 
     // 1. samples, anchor, running sums
     const gptr<const float> x = to_global(static_cast<const float *>(sg.x)) + base;
     const int nSamp = static_cast<int>(min(static_cast<long long>(SPAN), sg.n - base));
-    const float spread = x[min(lane * (SPAN / 64), nSamp - 1)];
+    const float spread = x[(lane * nSamp) >> 6];
     const int p0 = tid * SPT;
     float v[SPT];
 #pragma unroll

@@ -169,3 +169,19 @@ def test_sample_just_past_a_tile(variant, lt, bad):
         ref = O.pearson(t, clean)[:out[r].size]
         err = np.abs(out[r].astype(np.float64) - ref)[~touched]
         assert err.max() < 1e-5, (r, np.flatnonzero(~touched)[err.argmax()], err.max())
+
+
+@pytest.mark.parametrize("variant,lt,nfft", [(3, 200, 0), (4, 200, 0), (2, 300, 2048), (2, 300, 1024)])
+def test_last_sample_of_a_short_block_flags_no_block(variant, lt, nfft):
+    """A last sample of 200 times the noise in a short last block is one sample
+    of its anchor at most, and no reason to recompute the block's windows."""
+    rng = np.random.default_rng(83)
+    tpls = _templates(rng, (lt,) * 5)
+    step = ((nfft - lt + 1) & ~1) if nfft else 512
+    n = 5 * step + (nfft // 8 if nfft else 64) + lt
+    x = rng.standard_normal(n).astype(np.float32)
+    x[-1] = 200.0
+    out, ws = _rows(tpls, x, np.float32, nfft=nfft, variant=variant)
+    assert ws["flagged"] == 0, ws
+    for r, t in enumerate(tpls):
+        assert np.abs(out[r].astype(np.float64) - O.pearson(t, x)[:out[r].size]).max() < 1e-5, r

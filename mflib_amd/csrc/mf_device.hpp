@@ -241,6 +241,35 @@ __device__ __forceinline__ double read_lane(double v, int l)
                             __builtin_amdgcn_readlane(__double2loint(v), l));
 }
 
+// Largest value of the wave (lanes that a step leaves out keep their own).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_max(float v)
+{
+    const int i = __float_as_int(v);
+    return fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(i, i, CTRL, ROWS, 0xf, false)));
+}
+__device__ __forceinline__ float wave_max(float v)
+{
+    v = dpp_max<0x111, 0xf>(v);
+    v = dpp_max<0x112, 0xf>(v);
+    v = dpp_max<0x114, 0xf>(v);
+    v = dpp_max<0x118, 0xf>(v);
+    v = dpp_max<0x142, 0xa>(v);
+    v = dpp_max<0x143, 0xc>(v);
+    return read_lane(v, 63);
+}
+// Mean of a value per lane without the largest and the smallest of them (the
+// largest when nothing is left), the same on every lane: a single outlier does
+// not move it.
+__device__ __forceinline__ float wave_trimmed_mean(float v)
+{
+    const float hi = wave_max(v), lo = -wave_max(-v);
+    const bool in = !(v == hi || v == lo);
+    const int n = __popcll(__ballot(in));
+    const float mean = read_lane(wave_scan_sum(in ? v : 0.0f), 63) / static_cast<float>(n);
+    return uniform(n > 0 ? mean : hi);
+}
+
 // ---- block reductions -------------------------------------------------
 __device__ __forceinline__ double wave_sum(double v)
 {

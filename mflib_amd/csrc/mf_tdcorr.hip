@@ -169,8 +169,10 @@ struct TdBlock {
 };
 
 // Stages outputs [base, base + IS) of lane sg: loads the samples, takes the
-// anchor (the mean of 64 samples spread over the block, taken by every wave:
-// any value near the samples will do) and the RMS about it, splits x~ into
+// anchor (a mean of 64 samples spread over the block, taken by every wave: any
+// value near the samples will do; without the largest and the smallest, as a
+// glitch of 100 times the noise among them moved it far enough to make every
+// window of the item noisy) and the RMS about it, splits x~ into
 // its parts, builds the FP64 prefix sums and the equal-neighbour bits.  Each
 // thread takes consecutive samples and the scan runs on DPP moves, with one
 // barrier inside (the split by LDS copies of every entry, sums behind four
@@ -195,7 +197,7 @@ __device__ __forceinline__ TdBlock td_stage(TdStage<MT, KT> &sm, const Seg &sg, 
     for (int q = 0; q < SPT; ++q) { v[q] = p0 + q < nSamp ? x[p0 + q] : 0.0f; }
     const float after = p0 + SPT < nSamp ? x[p0 + SPT] : 0.0f;
     if (tid < (SPAN + 31) / 32) { sm.eqw[tid] = 0u; }
-    const double a = static_cast<double>(read_lane(wave_scan_sum(spread * (1.0f / 64)), 63));
+    const double a = static_cast<double>(wave_trimmed_mean(spread));
     double t1 = 0, t2 = 0;
     double l1[SPT], l2[SPT];  // exclusive sums inside the thread
 #pragma unroll

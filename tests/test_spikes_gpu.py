@@ -185,3 +185,19 @@ def test_last_sample_of_a_short_block_flags_no_block(variant, lt, nfft):
     assert ws["flagged"] == 0, ws
     for r, t in enumerate(tpls):
         assert np.abs(out[r].astype(np.float64) - O.pearson(t, x)[:out[r].size]).max() < 1e-5, r
+
+
+@pytest.mark.parametrize("variant,lt", [(3, 200), (4, 200), (3, 60), (4, 100)])
+def test_one_outlier_flags_no_item(variant, lt):
+    """A spike of 200 times the noise on a sample that a time-domain item takes
+    its anchor from is no reason to recompute the item's windows."""
+    rng = np.random.default_rng(89)
+    tpls = _templates(rng, (lt,) * 5)
+    kt = 256 if lt > 128 else 128 if lt > 64 else 64
+    n = 512 * 41 + lt
+    x = rng.standard_normal(n).astype(np.float32)
+    x[2_048 * np.arange(10) + 20 * (512 + kt) // 64] = 200.0
+    out, ws = _rows(tpls, x, np.float32, variant=variant)
+    assert ws["flagged"] == 0, ws
+    for r, t in enumerate(tpls):
+        assert np.abs(out[r].astype(np.float64) - O.pearson(t, x)[:out[r].size]).max() < 1e-5, r

@@ -426,28 +426,33 @@ __global__ __launch_bounds__(NT) void corr_kernel(const Item *__restrict__ items
             compute_scale<T, 16>(raw, ts1, ts2, tp1, tp2, sc, a, nValidSeg, Lt, noise, tid, NT);
             __syncthreads();
         }
-        // 4a. spectral product into Ws
-        const Cx<T> *H = static_cast<const Cx<T> *>(row.H);
-        for (int k = tid; k < M; k += NT) { Ws[k] = cmul(Xs[k], H[k]); }
+        // 4a. spectral product into Ws, the spectrum's loads all in flight
+        // together (in a loop each waited for the store before it)
+        const gptr<const Cx<T>> H = to_global(static_cast<const Cx<T> *>(row.H));
+        Cx<T> hk[SPT / 2];
+#pragma unroll
+        for (int q = 0; q < SPT / 2; ++q) { hk[q] = load_cx(H, tid + q * NT); }
+#pragma unroll
+        for (int q = 0; q < SPT / 2; ++q) { Ws[tid + q * NT] = cmul(Xs[tid + q * NT], hk[q]); }
         __syncthreads();
         // 4b. inverse FFT; Ws[n] W_{4M}^-n = c_n - i c_{n+M}
         fft_lds<T, M, NT, true>(Ws, tw);
         // 4c. normalisation epilogue
-        T *out = static_cast<T *>(row.out) + base;
-        const auto store = [&](int i, T c) {
-            if (i < nvRow) {
-                const T f = sc[i];
-                if (f >= T(0)) {
-                    T rho = c * f;
-                    if (fabs(rho) > T(1.1)) { rho = T(0); }
-                    out[i] = rho;
-                }
+        gptr<T> out = to_global(static_cast<T *>(row.out)) + base;
+        const auto store = [&](int i, T c, T f) {
+            if (i < nvRow && f >= T(0)) {
+                T rho = c * f;
+                if (fabs(rho) > T(1.1)) { rho = T(0); }
+                out[i] = rho;
             }
         };
-        for (int n = tid; n < M; n += NT) {
+#pragma unroll 2
+        for (int q = 0; q < SPT / 2; ++q) {
+            const int n = tid + q * NT;
+            const T f0 = sc[n], f1 = sc[n + M];  // past the row's end: not used
             const Cx<T> c = cmul(Ws[n], cconj(tw(n)));
-            store(n, c.x);
-            store(n + M, -c.y);
+            store(n, c.x, f0);
+            store(n + M, -c.y, f1);
         }
         // 4d. exact FP64 two-pass Pearson for flagged windows
         {

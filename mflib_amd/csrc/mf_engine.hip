@@ -347,7 +347,12 @@ void initialize(mf_handle *h)
     }
     // lanes: one per (channel, template-length bucket) carrying rows
     std::vector<std::vector<int>> chRows(nC);
-    for (int r = 0; r < nT; ++r) { chRows[rowCh[r]].push_back(r); }
+    std::vector<double> chOut(nC, 0.0);  // outputs of a channel's longest row
+    for (int r = 0; r < nT; ++r) {
+        chRows[rowCh[r]].push_back(r);
+        chOut[rowCh[r]] = std::max(chOut[rowCh[r]], static_cast<double>(h->rows[r].nOut));
+    }
+    const double allOut = std::accumulate(chOut.begin(), chOut.end(), 0.0);
     for (int c = 0; c < nC; ++c) {
         if (chRows[c].empty()) { continue; }
         std::vector<int> sorted = chRows[c];
@@ -386,7 +391,7 @@ void initialize(mf_handle *h)
             outs.erase(outs.begin(), outs.begin() + nTd);
             if (sorted.empty()) { continue; }
         }
-        for (const Bucket &bk : planBuckets(h->precision, h->userNfft == 0 ? 0 : h->userNfft, lts, outs)) {
+        for (const Bucket &bk : planBuckets(h->precision, h->userNfft, lts, outs, allOut / chOut[c])) {
             mf_handle::Lane ln;
             ln.ch = c;
             ln.mix = bk.mix;

@@ -450,10 +450,25 @@ inline double spectrumPenalty(int precision, int logM, long long rows, double ro
     return rowBlocks * specBytes / 4.0e12 * 1.0e6;  // microseconds
 }
 
+// The cost tables hold a block's share of a full GPU's time.  A launch of
+// fewer blocks than compute units takes the time of one block, however few
+// there are: the factor of its blocks' summed cost.  `lanes` is the number of
+// lanes like this one that run together (their outputs over this lane's); 0 for
+// a lane among unknown many others, as in the server's batches, which counts as
+// a full GPU.  One channel of 100,000 samples with 20 templates of 367 to 500
+// samples, in FP64, an apply: 91 us in 64 blocks of 2048, 69 us in 191 of 1024;
+// with 20 templates of 867 to 1000 in FP32: 98 us in 32 blocks of 4096, 61 us in
+// 95 of 2048; a full GPU prefers the larger blocks in both.
+constexpr double kComputeUnits = 256;
+inline double fillFactor(double blocks, double lanes)
+{
+    return lanes > 0 ? std::max(1.0, kComputeUnits / (blocks * lanes)) : 1.0;
+}
+
 // Predicted cost of a lane for an FFT size and a variant (0 = the default
 // variant), or -1 if the plan is impossible: blocks x the per-block part
 // plus row blocks x the per-row part.
-inline double laneCost(int precision, int logM, int variant, const LaneRows &rs)
+inline double laneCost(int precision, int logM, int variant, const LaneRows &rs, double lanes)
 {
     const long long N = 2LL << logM;
     const long long L = N - rs.nb() + 1;
@@ -462,6 +477,7 @@ inline double laneCost(int precision, int logM, int variant, const LaneRows &rs)
     double shared = 0, solo = 0;
     laneRowBlocks(rs, L, shared, solo);
     const double penalty = spectrumPenalty(precision, logM, static_cast<long long>(rs.Lt.size()), shared + solo);
+    const double factor = blockRisk(logM) * fillFactor(blocks, lanes);
     std::lock_guard<std::mutex> lk(costMutex());
     const CostTable &t = costTable(precision);
     if (t.measured) {
@@ -473,15 +489,14 @@ inline double laneCost(int precision, int logM, int variant, const LaneRows &rs)
                 const double c = blocks * t.a[logM][cand] + t.bShared[logM][cand] * shared + t.bSolo[logM][cand] * solo;
                 if (best < 0 || c < best) { best = c; v = cand; }
             }
-            if (best >= 0) { return best * blockRisk(logM) + penalty; }
+            if (best >= 0) { return best * factor + penalty; }
         } else if (t.a[logM][v] > 0) {
-            return (blocks * t.a[logM][v] + t.bShared[logM][v] * shared + t.bSolo[logM][v] * solo) * blockRisk(logM) +
-                   penalty;
+            return (blocks * t.a[logM][v] + t.bShared[logM][v] * shared + t.bSolo[logM][v] * solo) * factor + penalty;
         }
     }
     // static model: per-block part and per-row parts at the same scale
     const double unit = staticBlockCost(logM, RowMix{0, 0}, precision);
-    return unit * (blocks + 1.15 * shared + 1.84 * solo) * blockRisk(logM) + penalty;
+    return unit * (blocks + 1.15 * shared + 1.84 * solo) * factor + penalty;
 }
 
 // Correlation kernel variant of one lane: a requested variant if it exists
@@ -510,7 +525,7 @@ inline int laneVariant(int precision, int logM, int requested, RowMix mix)
 // FFT size (as logM, nfft = 2^(logM+1)) of a lane whose longest template
 // has nb samples and which produces nOut outputs for the rows in `mix`.  A
 // positive userNfft forces the size.
-inline int chooseLogM(int precision, int userNfft, const LaneRows &rs)
+inline int chooseLogM(int precision, int userNfft, const LaneRows &rs, double lanes)
 {
     const int nb = rs.nb();
     const int hiLog = maxLogM(precision);
@@ -534,7 +549,7 @@ inline int chooseLogM(int precision, int userNfft, const LaneRows &rs)
     for (int lg = mfk::kMinLogM; lg <= hiLog; ++lg) {
         const long long N = 2LL << lg;
         if (N - nb + 1 < N / 4 && lg < hiLog) { continue; }  // keep >= 25% useful outputs
-        const double c = laneCost(precision, lg, 0, rs);
+        const double c = laneCost(precision, lg, 0, rs, lanes);
         if (c < 0) { continue; }
         if (best < 0 || c < bestCost) { best = lg; bestCost = c; }
     }
@@ -577,7 +592,7 @@ inline LaneRows laneRows(const std::vector<int> &sortedLt, const std::vector<lon
 }
 
 inline Bucket makeBucket(int precision, int userNfft, const std::vector<int> &sortedLt,
-                         const std::vector<long long> &nOut, int begin, int end)
+                         const std::vector<long long> &nOut, int begin, int end, double lanes)
 {
     Bucket b;
     b.begin = begin;
@@ -585,18 +600,18 @@ inline Bucket makeBucket(int precision, int userNfft, const std::vector<int> &so
     b.nb = sortedLt[end - 1];
     const LaneRows rs = laneRows(sortedLt, nOut, begin, end);
     b.mix = rs.mix();
-    b.logM = chooseLogM(precision, userNfft, rs);
-    b.cost = laneCost(precision, b.logM, 0, rs);
+    b.logM = chooseLogM(precision, userNfft, rs, lanes);
+    b.cost = laneCost(precision, b.logM, 0, rs, lanes);
     return b;
 }
 
 // sortedLt: the channel's template lengths in increasing order; nOut[i]:
-// the outputs of row i of that order.
+// the outputs of row i of that order; lanes: see fillFactor.
 inline std::vector<Bucket> planBuckets(int precision, int userNfft, const std::vector<int> &sortedLt,
-                                       const std::vector<long long> &nOut)
+                                       const std::vector<long long> &nOut, double lanes)
 {
     const int n = static_cast<int>(sortedLt.size());
-    if (userNfft > 0 || n <= 1) { return {makeBucket(precision, userNfft, sortedLt, nOut, 0, n)}; }
+    if (userNfft > 0 || n <= 1) { return {makeBucket(precision, userNfft, sortedLt, nOut, 0, n, lanes)}; }
     // Optimal split into contiguous buckets by dynamic programming over the
     // boundaries between runs of equal length (a run stays in one bucket, so
     // its rows keep sharing a scale): best[J] = min over I < J and FFT size
@@ -634,7 +649,7 @@ inline std::vector<Bucket> planBuckets(int precision, int userNfft, const std::v
             const double unit = staticBlockCost(lg, RowMix{0, 0}, precision);
             best = unit * (blocks + 1.15 * sS + 1.84 * sO);
         }
-        return best * blockRisk(lg) + spectrumPenalty(precision, lg, rows, sS + sO);
+        return best * blockRisk(lg) * fillFactor(blocks, lanes) + spectrumPenalty(precision, lg, rows, sS + sO);
     };
     std::vector<double> best(R + 1, -1);
     std::vector<int> fromRun(R + 1, -1), fromLog(R + 1, -1);
@@ -679,7 +694,7 @@ inline std::vector<Bucket> planBuckets(int precision, int userNfft, const std::v
         const LaneRows rs = laneRows(sortedLt, nOut, b.begin, b.end);
         b.mix = rs.mix();
         b.logM = fromLog[J];
-        b.cost = laneCost(precision, b.logM, 0, rs);
+        b.cost = laneCost(precision, b.logM, 0, rs, lanes);
         bk.push_back(b);
     }
     std::reverse(bk.begin(), bk.end());

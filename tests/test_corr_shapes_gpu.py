@@ -219,3 +219,18 @@ def test_device_signal_of_almost_2_31_samples():
     got = h.get_signal(0, n)[-4:]
     assert np.array_equal(got, np.array([0.0, 1.0, -2.0, 0.5], dtype=np.float32))
     h.close()
+
+
+def test_plans_of_few_and_of_many_blocks():
+    """FP64 rows of 400 to 500 samples: blocks of 2048 where they fill the
+    device, blocks of 1024 where fewer blocks than compute units are all the
+    work there is (a launch then takes one block's time)."""
+    rng = np.random.default_rng(25)
+    tpls = [rng.standard_normal(L) for L in range(400, 500, 5)]
+    for n, nfft in ((100_000, 1024), (8_000_000, 2048)):
+        h = capi.Handle(np.float64, "batched")
+        h.set_templates(tpls)
+        h.set_batch_layout([n], [0] * len(tpls), [0] * len(tpls), 1)
+        h.initialize()
+        assert {h.plan(r)[0] for r in range(len(tpls))} == {nfft}, n
+        h.close()

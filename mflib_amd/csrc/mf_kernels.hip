@@ -124,21 +124,38 @@ __device__ __forceinline__ void window_sums(const T *raw, const double *ts1, con
     const int q0 = (lo + TILE - 1) / TILE, q1 = hi / TILE;
     S1 = 0;
     S2 = 0;
+    if constexpr (sizeof(T) == 8) {
+        // the same sums in the same order, four reads in flight: a row's only
+        // serial chain of LDS round trips, tens of them for a long template
+        const auto samples = [&](int from, int to) {
+#pragma unroll 4
+            for (int j = from; j < to; ++j) {
+                const double d = static_cast<double>(raw[j]) - a;
+                S1 += d;
+                S2 += d * d;
+            }
+        };
+        if (q0 < q1) {
+            samples(lo, TILE * q0);
+#pragma unroll 4
+            for (int q = q0; q < q1; ++q) {
+                S1 += ts1[q];
+                S2 += ts2[q];
+            }
+            samples(TILE * q1, hi);
+        } else {
+            samples(lo, hi);
+        }
+        return;
+    }
     if (q0 < q1) {
         for (int j = lo; j < TILE * q0; ++j) {
             const double d = static_cast<double>(raw[j]) - a;
             S1 += d;
             S2 += d * d;
         }
-        if constexpr (sizeof(T) == 4) {
-            S1 += tp1[q1] - tp1[q0];
-            S2 += tp2[q1] - tp2[q0];
-        } else {
-            for (int q = q0; q < q1; ++q) {
-                S1 += ts1[q];
-                S2 += ts2[q];
-            }
-        }
+        S1 += tp1[q1] - tp1[q0];
+        S2 += tp2[q1] - tp2[q0];
         for (int j = TILE * q1; j < hi; ++j) {
             const double d = static_cast<double>(raw[j]) - a;
             S1 += d;

@@ -567,10 +567,13 @@ void initialize(mf_handle *h)
                 }
                 const int nRows = static_cast<int>(ln.rows.size());
                 // An item stages its samples once for all its rows, and its four
-                // waves take 16 rows at a time: about 128 rows an item, evenly
-                // (150 rows in one item instead of 128 + 22: 0.98 against
-                // 1.15 ms; 256 in two instead of one: 2.38 against 2.44 ms).
-                const int parts = std::max(1, (nRows + 64) / 128);
+                // waves take 16 rows at a time, 64 rows in all: one item up to
+                // 192 rows, then about 128 rows an item, evenly.  4 channels x 1 M
+                // samples, 200 taps, in one item / in two, FP16 and BF16 us: 144
+                // rows 1197/1425 and 1749/2265, 192 rows 1397/1562 and 2107/2414,
+                // 208 rows 1604/1619 and 2441/2513, 224 rows 1709/1668 and
+                // 2593/2649, 256 rows 1847/1840 and 2878/2817.
+                const int parts = std::max(1, (nRows + 63) / 128);
                 const int rowsPerItem = (nRows + 16 * parts - 1) / (16 * parts) * 16;
                 for (long long s0 = 0; s0 < ln.nOut; s0 += mfk::kTdOutputsPerItem) {
                     for (int g = 0; g < nRows; g += rowsPerItem) {

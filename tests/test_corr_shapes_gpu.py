@@ -234,3 +234,13 @@ def test_plans_of_few_and_of_many_blocks():
         h.initialize()
         assert {h.plan(r)[0] for r in range(len(tpls))} == {nfft}, n
         h.close()
+
+
+@pytest.mark.parametrize("rows", [192, 193])
+def test_time_domain_rows_on_either_side_of_the_item_split(rows):
+    """192 rows are one item, 193 two of 112 and 81."""
+    rng = np.random.default_rng(27)
+    lengths = tuple(int(v) for v in rng.integers(20, 129, size=rows))
+    for variant in (3, 4):
+        _, out, ref = _rows(lengths, 1_500, np.float32, 0, variant)
+        _check(out, ref, 1e-5, (variant, rows))

@@ -283,7 +283,10 @@ inline std::mutex &costMutex()
 }
 
 // mf_autotune's measurements on an MI355X (microseconds per block for the
-// whole GPU; variant 1 block-wide, 2 wave-level).
+// whole GPU; variant 1 block-wide, 2 wave-level).  The largest block-wide
+// entries have since become up to a fifth cheaper (FP32 12: 0.086, 0.049,
+// 0.065; FP64 11: 0.053, 0.033, 0.056); plans from a table measured anew were
+// no better (mixed requests 10.66 -> 10.97 ms, 270 small shapes 0.997 times).
 inline CostTable defaultCostTable(int precision)
 {
     CostTable t;
@@ -438,14 +441,14 @@ constexpr double kBlockRisk = 0.5;
 inline double blockRisk(int logM) { return 1.0 + kBlockRisk * (logM - mfk::kMinLogM); }
 
 // Extra cost of a lane whose template spectra do not stay in its XCD's L2
-// (4 MB): each row block then streams its row's spectrum, (M + 1) complex
+// (4 MB): each row block then streams its row's spectrum, M complex
 // values, from the MALL or HBM, priced at 4 TB/s for the whole GPU (half the
 // HBM peak: the reads compete with the rho writes).  The autotuner's
 // synthetic lanes (8 rows) never reach this, so the term is added on top.
 inline double spectrumPenalty(int precision, int logM, long long rows, double rowBlocks)
 {
     constexpr double kL2Budget = 3.0 * (1 << 20);
-    const double specBytes = static_cast<double>((1LL << logM) + 1) * 2.0 * (precision == MF_PRECISION_FLOAT ? 4 : 8);
+    const double specBytes = static_cast<double>(1LL << logM) * 2.0 * (precision == MF_PRECISION_FLOAT ? 4 : 8);
     if (static_cast<double>(rows) * specBytes <= kL2Budget) { return 0.0; }
     return rowBlocks * specBytes / 4.0e12 * 1.0e6;  // microseconds
 }
@@ -472,7 +475,7 @@ inline double laneCost(int precision, int logM, int variant, const LaneRows &rs,
 {
     const long long N = 2LL << logM;
     const long long L = N - rs.nb() + 1;
-    if (L < 2) { return -1; }  // even block starts need L >= 2
+    if (L < 2) { return -1; }  // an even block length needs L >= 2
     const double blocks = std::ceil(static_cast<double>(rs.maxOut()) / static_cast<double>(L));
     double shared = 0, solo = 0;
     laneRowBlocks(rs, L, shared, solo);
@@ -561,8 +564,8 @@ inline int chooseLogM(int precision, int userNfft, const LaneRows &rs, double la
     return best;
 }
 
-// Block length of a lane: nfft - nb + 1, made even so that every block
-// start stays 8-byte aligned for the paired stores of the epilogue.
+// Block length of a lane: nfft - nb + 1, made even (every FP32 block then
+// starts at an 8-byte boundary of its row).
 inline int blockLength(int logM, int nb)
 {
     int L = static_cast<int>((2LL << logM) - nb + 1);

@@ -1,8 +1,11 @@
 // Matched-filter kernels for gfx950 (MI355X, CDNA4, wave64).
 //
-// corr_kernel  -- the hot path.  One block = one FFT block of one channel
-//   lane; it serves every template row on that channel:
-//     1. load nfft samples (coalesced), FP64 block anchor (window mean),
+// corr2_kernel -- the hot path up to nfft 4096 (FP32) and 2048 (FP64): the
+//   steps below on wave-level FFTs, see there.
+// corr_kernel  -- the block-wide form, for the larger FFT sizes and for lanes of
+//   few rows.  One block = one FFT block of one channel lane; it serves every
+//   template row on that channel:
+//     1. load nfft samples (coalesced), FP64 block anchor (their mean),
 //        FP64 16-sample tile sums of (x-a) and (x-a)^2 via wave shuffles;
 //     2. forward transform of the anchored block modulo z^M + i (see
 //        mf_device.hpp), kept in LDS for all rows;
@@ -44,7 +47,9 @@ constexpr int NT = kThreads;
 // times sqrt(Lt), templates of 200-2000 samples, nfft 2048/4096), the worst
 // error was 1.47x the bound and 4.5e-7 absolute.  The FP32 tolerance of
 // 2.5e-6 therefore keeps unflagged windows below ~4e-6, inside the 1e-5
-// contract; FP64 correlation keeps 1e-12.
+// contract; FP64 correlation keeps 1e-12, up to 2e-11 in the windows that a
+// spike of 1e4 times the noise has just left (the sliding sums keep 2^-53 of
+// its square).
 template <typename T>
 struct Eps;
 template <>

@@ -303,7 +303,7 @@ __device__ __forceinline__ void td_dead(const TdItem &item, const TdRow *__restr
 // split taps of 16 rows (parts * KT / 8 VGPRs: 96 for the BF16 triple at
 // KT = 256; tiles of 32 rows would need 192 and leave one wave per SIMD)
 // and walks the item's 32 output tiles; the 4 waves take 64 rows at a
-// time, in two row groups when the item has more.  A lane holds column
+// time, in up to three row groups.  A lane holds column
 // i = lane % 16 and rows 4 (lane / 16) + r, r = 0..3: their epilogue
 // constants stay in registers for the row group, and each quarter wave
 // stores 16 consecutive outputs of its row.

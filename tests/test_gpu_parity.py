@@ -534,10 +534,10 @@ def test_time_domain_short_tap_lanes_match_oracle(variant):
 
 @pytest.mark.parametrize("variant", [3, 4])
 def test_time_domain_many_rows_per_lane_match_oracle(variant):
-    """150 short templates of 20-256 taps on one channel: work items of 128
-    and 22 rows, so every wave of a block holds a partial or empty row set
-    and the 16-row tiles take two row groups; every row within the FP32
-    contract of the FP64 oracle."""
+    """150 short templates of 20-256 taps on one channel: one work item whose
+    rows take three groups of 64, the last of them partial (a wave with 16
+    rows, one with 6 and two with none); every row within the FP32 contract of
+    the FP64 oracle."""
     rng = np.random.default_rng(740 + variant)
     n = 6_000
     x = (rng.standard_normal(n) * 2 + 300.0).astype(np.float32)

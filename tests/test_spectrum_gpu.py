@@ -2,12 +2,13 @@
 
 The reference returns row `it` of mB: the r2c transform of the demeaned,
 unit-norm, time-reversed template zero-padded to nfft
-(src/matchedFilter.cpp:556-620).  The engine keeps conj(T^)/(2 nfft) of the
-unreversed template and rebuilds the export with a phase rotation and a
-rescale; this checks that rebuild against the oracle's own FFT of the
-oracle's reversed template at the engine's nfft.  A wrong sign, offset or
-scale fails it: the phase of bin k carries the template length, so a
-non-power-of-two length and an off-by-one in Lt both show."""
+(src/matchedFilter.cpp:556-620).  The engine's own spectra are at other
+frequencies, so the export transforms the FP64 taps that the engine prepared;
+this checks it against the oracle's own FFT of the oracle's reversed template
+at the engine's nfft.  A wrong sign, offset or scale fails it: the phase of bin
+k carries the template length, so a non-power-of-two length and an off-by-one
+in Lt both show.  The engine's own spectra are checked by the correlations of
+every other test."""
 import numpy as np
 import pytest
 

@@ -507,7 +507,7 @@ __global__ __launch_bounds__(NT, kTdBlocks) void tdcorr_kernel(const TdItem *__r
 #pragma unroll
                         for (int r = 0; r < 4; ++r) {
                             const bool flag = i < nvR[r] && ((flags[r] >> lane) & 1u);
-                            const bool flat = flag && run > 0 && run >= LtR[r] - 1;
+                            const bool flat = flag && run >= LtR[r] - 1;  // a one-sample window always
                             if (flat) { outR[r][i] = 0.0f; }
                             const unsigned nFlat = static_cast<unsigned>(__popcll(__ballot(flat)));
                             nFlag += nFlat;

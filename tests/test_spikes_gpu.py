@@ -201,3 +201,15 @@ def test_one_outlier_flags_no_item(variant, lt):
     assert ws["flagged"] == 0, ws
     for r, t in enumerate(tpls):
         assert np.abs(out[r].astype(np.float64) - O.pearson(t, x)[:out[r].size]).max() < 1e-5, r
+
+
+@pytest.mark.parametrize("variant", [3, 4])
+def test_time_domain_one_sample_templates(variant):
+    """A window of one sample is constant, so 0, also where the sample is a NaN
+    or an infinity."""
+    rng = np.random.default_rng(97)
+    x = rng.standard_normal(1_300).astype(np.float32)
+    x[[3, 600]] = np.nan, np.inf
+    out, _ = _rows([np.array([1.0]), np.array([1.0, -1.0])], x, np.float32, variant=variant)
+    assert not out[0].any()
+    assert np.isnan(out[1][2:4]).all()
